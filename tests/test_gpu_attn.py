@@ -1,0 +1,101 @@
+"""GPU tests of the attention kernels' dispatch edges (csrc/uq_attn.hip):
+softmax rows around every row-kernel size, outputs that sit on f32 rounding
+midpoints (the reference's sequential sum replayed by a workgroup), and the
+prefill's tile kernels against single-query steps over long caches. Every
+comparison is bit for bit: the kernels' contract is the reference's own bits.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import uq
+from uq import layer as L
+from uq import ops
+from test_gpu_layers import SMALL, Model
+from test_gpu_ops import assert_bitwise, check_attn, softmax_model
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,rows", [(1, 3), (255, 2), (1024, 2), (1025, 2), (4096, 2), (4097, 2), (8193, 2),
+                                    (16385, 2), (32768, 2), (32769, 2), (1500, 600), (2049, 600), (4095, 600)])
+def test_softmax_rows_at_the_row_kernels_edges(n, rows):
+    rng = np.random.default_rng(n + rows)
+    X = rng.standard_normal((rows, n)).astype(np.float32) * 5
+    d = uq.DeviceArray.from_numpy(X)
+    ops.softmax_d(d, d, n, rows, 0.5)
+    uq.synchronize()
+    got = d.download(np.float32, rows * n).reshape(rows, n)
+    for r in {0, 1, rows - 1}:
+        assert_bitwise(got[r], softmax_model(X[r], 0.5), f"softmax n={n} row {r}")
+
+
+def midpoint_column(rng, n, w):
+    """n f32 values whose sum of w v in position order is within an f64 ulp or
+    two of the midpoint of two f32 values: ever smaller values close the gap."""
+    v = rng.standard_normal(n).astype(np.float32)
+    v[-6:] = 0.0
+    s = float(np.add.accumulate(w * v.astype(np.float64))[-1])
+    lo = np.float32(s)
+    mid = (float(lo) + float(np.nextafter(lo, np.float32(np.inf)))) / 2
+    for k in range(n - 6, n):
+        v[k] = np.float32((mid - s) / w)
+        s = float(np.add.accumulate(w * v.astype(np.float64))[-1])
+    assert abs(s - mid) <= 4 * np.spacing(abs(mid)), "the column does not reach the midpoint"
+    return v
+
+
+@pytest.mark.parametrize("n_ctx", [40, 1000, 5000, 20000])
+@pytest.mark.parametrize("cols", [(5,), (0, 1, 17, 18, 63), tuple(range(16, 27))])
+def test_attn_decode_outputs_on_midpoints(n_ctx, cols):
+    """Equal weights, value columns planted on f32 midpoints: no bound decides
+    them. One, a few (a workgroup replays each) and eleven of one workgroup's
+    columns (each lane its own)."""
+    hd = 64
+    rng = np.random.default_rng(n_ctx + len(cols))
+    w = float(O.softmax(np.zeros(n_ctx, np.float32), 1.0)[0])
+    vc = rng.standard_normal((n_ctx, hd)).astype(np.float32)
+    for c in cols:
+        vc[:, c] = midpoint_column(rng, n_ctx, w)
+    check_attn(np.ones(hd, np.float32), np.ones(n_ctx * hd, np.float32), vc.reshape(-1), n_ctx, 1, 1, hd, 1.0,
+               f"midpoints n={n_ctx}", bit_exact_soft=True)
+
+
+def attn_layer(m, X, K, V, n_ctx_max, pos0, prefill):
+    d, (nt, n) = m.d, X.shape
+    kc, vc, dx, dl = (uq.DeviceArray.from_numpy(a) for a in (K, V, X, np.zeros_like(X)))
+    ws = uq.DeviceArray(4 * max(L.ws_floats(d, n_ctx_max), L.prefill_ws_floats(d, nt, attn=m.aw, n_ctx_max=n_ctx_max)))
+    out = np.empty_like(X)
+    if prefill:
+        L.attn_prefill(d, m.aw, kc, vc, n_ctx_max, pos0, nt, dx, dl, ws)
+        out = dl.download(np.float32, nt * n).reshape(nt, n)
+    else:
+        for t in range(nt):
+            one = uq.DeviceArray.from_numpy(X[t])
+            L.attn_step(d, m.aw, kc, vc, n_ctx_max, pos0 + t, one, dl, ws)
+            out[t] = dl.download(np.float32, n)
+            one.free()
+    for a in (kc, vc, dx, dl, ws):
+        a.free()
+    return out
+
+
+@pytest.mark.parametrize("shape,nt,pos0", [
+    (dict(n_head=8, n_head_kv=2, head_dim=64), 3, 1700),  # queries by themselves
+    (dict(n_head=8, n_head_kv=2, head_dim=64), 90, 1009),  # scores in tiles, values by themselves
+    (dict(n_head=8, n_head_kv=2, head_dim=64), 333, 29),  # both in tiles
+    (dict(n_embd=1280, n_v_heads=20, n_head=5, n_head_kv=1, head_dim=256), 65, 1100),  # group 5
+    (dict(n_embd=768, n_v_heads=12, n_head=6, n_head_kv=2, head_dim=128), 130, 2051),  # group 3
+    (dict(n_head=1, n_head_kv=1, head_dim=512, n_rot=32), 140, 600)])  # scores by themselves, values in tiles
+def test_attn_prefill_over_a_long_cache_equals_steps(shape, nt, pos0):
+    m = Model(dict(SMALL, **shape), seed=71 + nt)
+    c = m.cfg
+    rng = np.random.default_rng(nt + pos0)
+    n_ctx_max = pos0 + nt + 3
+    K, V = (rng.standard_normal(n_ctx_max * c.n_head_kv * c.head_dim).astype(np.float32) for _ in range(2))
+    X = rng.standard_normal((nt, c.n_embd)).astype(np.float32)
+    ref = attn_layer(m, X, K, V, n_ctx_max, pos0, False)
+    got = attn_layer(m, X, K, V, n_ctx_max, pos0, True)
+    for t in range(nt):
+        assert_bitwise(got[t], ref[t], f"attn {shape} token {t} of {nt} at {pos0}")
+    m.free()

@@ -93,6 +93,9 @@ __device__ __forceinline__ void q8k_replay(const uint32_t *rr, int nblk, int k, 
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float expf_cr(float v) { return (float)exp((double)v); }
 
+// sigmoid (kernels.rs:198-203)
+__device__ __forceinline__ float sigmoid1(float v) { return __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_cr(-v))); }
+
 __device__ __forceinline__ float swiglu1(float g, float u) {
     return __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf_cr(-g))), u);
 }

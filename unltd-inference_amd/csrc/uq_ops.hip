@@ -27,19 +27,7 @@ constexpr int OPS_TPB = 256;
 
 __device__ __forceinline__ float logf_cr(float v) { return (float)log((double)v); }
 
-__device__ float block_max_f(float v, float *red) {
-    for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    float t = red[0];
-    for (int i = 1; i < (int)(blockDim.x >> 6); i++) t = fmaxf(t, red[i]);
-    __syncthreads();
-    return t;
-}
-
-// sigmoid (kernels.rs:198-203), silu (:207-212), softplus (:217-228)
-__device__ __forceinline__ float sigmoid1(float v) { return __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_cr(-v))); }
+// silu (kernels.rs:207-212), softplus (:217-228)
 __device__ __forceinline__ float silu1(float v) { return __fdiv_rn(v, __fadd_rn(1.0f, expf_cr(-v))); }
 __device__ __forceinline__ float softplus1(float v) { return v > 20.0f ? v : logf_cr(__fadd_rn(1.0f, expf_cr(v))); }
 
@@ -156,111 +144,6 @@ __global__ __launch_bounds__(OPS_TPB) void l2norm_kernel(float *__restrict__ dat
     const float sum32 = seq_sum_f32<OPS_TPB>([r](int i) { return r[i]; }, dim, S, [](double v) { return (float)v; }, &bc);
     const float scale = __fdiv_rn(1.0f, fmaxf(sqrtf_cr(sum32), eps));
     for (int i = threadIdx.x; i < dim; i += OPS_TPB) r[i] = __fmul_rn(r[i], scale);
-}
-
-// Pairwise tree (kernels.rs:27-42) of lv[0, len) in LDS, level by level:
-// pairs (2i, 2i+1), an odd tail carried up. Every thread takes part;
-// returns lv[0] to all (len <= 2 * OPS_TPB * kTreeRegs).
-constexpr int kTreeRegs = 16;
-__device__ double lds_tree(double *lv, int len) {
-    while (len > 1) {
-        const int nl = (len + 1) / 2;
-        double v[kTreeRegs];
-        int c = 0;
-        for (int p = threadIdx.x; p < nl; p += OPS_TPB, c++) v[c] = 2 * p + 1 < len ? lv[2 * p] + lv[2 * p + 1] : lv[2 * p];
-        __syncthreads();
-        c = 0;
-        for (int p = threadIdx.x; p < nl; p += OPS_TPB, c++) lv[p] = v[c];
-        __syncthreads();
-        len = nl;
-    }
-    const double r = lv[0];
-    __syncthreads();
-    return r;
-}
-
-// softmax (kernels.rs:157-168), one workgroup per row, in place allowed.
-// The denominator is pairwise_sum_f64 over the row. For a chunk size C that
-// is a power of two, level log2(C) of that tree holds the trees of the full
-// C-chunks followed by the tree of the remainder (whose node is always the
-// carried odd tail below that level), so the row sum is the pairwise tree
-// over the chunk sums: each chunk is reduced in LDS, then the chunk sums.
-constexpr int kSmChunk = 2 * OPS_TPB * kTreeRegs;  // 8192
-constexpr int kSmMaxChunks = 2048;
-static_assert((kSmChunk & (kSmChunk - 1)) == 0, "chunk trees must be nodes of the row tree");
-// Rows of token z = blockIdx.y (the attention of a prefill) are n + z dn
-// long and start zst floats after token z - 1's.
-__global__ __launch_bounds__(OPS_TPB) void softmax_kernel(float *out, const float *x, int n, float scale, int dn,
-                                                          size_t zst) {
-    __shared__ double lv[kSmChunk / 2];
-    __shared__ double cs[kSmMaxChunks];
-    __shared__ float red[OPS_TPB / 64];
-    n += (int)blockIdx.y * dn;
-    const size_t row0 = (size_t)blockIdx.y * zst + (size_t)blockIdx.x * n;
-    const float *xr = x + row0;
-    float *yr = out + row0;
-    float m = -INFINITY;
-    for (int i = threadIdx.x; i < n; i += OPS_TPB) m = fmaxf(m, xr[i]);
-    m = block_max_f(m, red);
-    auto ex = [&](int i) { return expf_cr(__fmul_rn(__fsub_rn(xr[i], m), scale)); };
-    const int nch = (n + kSmChunk - 1) / kSmChunk;
-    for (int c = 0; c < nch; c++) {
-        const int base = c * kSmChunk, cl = min(kSmChunk, n - base);
-        const int len = (cl + 1) / 2;  // level 1 straight from the exponentials
-        for (int p = threadIdx.x; p < len; p += OPS_TPB) {
-            const int i = base + 2 * p;
-            lv[p] = 2 * p + 1 < cl ? (double)ex(i) + (double)ex(i + 1) : (double)ex(i);
-        }
-        __syncthreads();
-        const double t = lds_tree(lv, len);
-        if (threadIdx.x == 0) cs[c] = t;
-    }
-    __syncthreads();
-    const double sum = lds_tree(cs, nch);
-    for (int i = threadIdx.x; i < n; i += OPS_TPB) yr[i] = (float)((double)ex(i) / sum);
-}
-
-// softmax_kernel for rows of at most kSmWaveMax (the attention of a short
-// context or of a prefill chunk): one wave per row, four rows a workgroup,
-// no barrier. Lane l holds elements [16 l, 16 l + 16); the row's pairwise
-// tree (kernels.rs:21-42) is the lanes' 16-element trees, then the wave's
-// fixed tree over the lanes (wave_sum_d), with the missing elements as
-// zeros: every term is an exponential (>= +0), so a zero added where the
-// tree carries an odd tail up leaves the same value. Row r of token z =
-// blockIdx.y (r < nr) is n + z dn long, token z's rows start zst floats
-// after token z - 1's.
-constexpr int kSmWaveMax = 1024;
-__global__ __launch_bounds__(OPS_TPB) void softmax_wave_kernel(float *out, const float *x, int n, float scale, int dn,
-                                                               size_t zst, int nr) {
-    const int lane = threadIdx.x & 63, r = blockIdx.x * (OPS_TPB / 64) + (int)(threadIdx.x >> 6);
-    if (r >= nr) return;  // the whole wave
-    n += (int)blockIdx.y * dn;
-    const size_t row0 = (size_t)blockIdx.y * zst + (size_t)r * n;
-    const float *xr = x + row0;
-    float *yr = out + row0;
-    const int i0 = 16 * lane;
-    float v[16];
-    float m = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-        v[k] = i0 + k < n ? xr[i0 + k] : -INFINITY;
-        m = fmaxf(m, v[k]);
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-#pragma unroll
-    for (int k = 0; k < 16; k++) v[k] = i0 + k < n ? expf_cr(__fmul_rn(__fsub_rn(v[k], m), scale)) : 0.0f;
-    double t[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) t[k] = (double)v[2 * k] + (double)v[2 * k + 1];
-#pragma unroll
-    for (int w = 4; w >= 1; w >>= 1)
-#pragma unroll
-        for (int k = 0; k < w; k++) t[k] = t[2 * k] + t[2 * k + 1];
-    const double sum = wave_sum_d(t[0]);
-#pragma unroll
-    for (int k = 0; k < 16; k++)
-        if (i0 + k < n) yr[i0 + k] = (float)((double)v[k] / sum);
 }
 
 // sigmoid, silu, softplus, gelu_tanh (kernels.rs:185-194)
@@ -738,455 +621,6 @@ __global__ __launch_bounds__(OPS_TPB) void matmul_acc_kernel(float *__restrict__
     if ((threadIdx.x & 63) == 0) acc[o] = (float)((double)acc[o] + s);
 }
 
-// ---- decode attention (qwen35_forward.rs:639-671) ----
-// Caches are [n_ctx][n_head_kv][hd] f32; q head h reads kv head h / group
-// (group = n_head / n_head_kv, consecutive heads share a kv head).
-
-// Pairwise sum (kernels.rs:21-42) of 64 * E values, lane l holding values
-// [E*l, E*l + E). For a power-of-two count the tree adds adjacent nodes
-// level by level: the lane-local tree, then the xor butterfly over lanes
-// (both lanes of a pair form the same node: f64 addition is commutative).
-template <int E>
-__device__ double wave_pairwise(double (&t)[E]) {
-#pragma unroll
-    for (int w = E; w > 1; w /= 2)
-#pragma unroll
-        for (int j = 0; j < w / 2; j++) t[j] = t[2 * j] + t[2 * j + 1];
-    double s = t[0];
-#pragma unroll
-    for (int off = 1; off < 64; off *= 2) s = s + __shfl_xor(s, off);
-    return s;
-}
-
-constexpr int kAttnMaxGroup = 8;
-constexpr int kScoresPPB = 8;  // positions per workgroup (2 per wave)
-
-// scores[h][p] = (f32) dot_f32(q_h, K[p][kv]) for the group's heads; one
-// wave per position, E = hd / 64 values per lane. Query z = blockIdx.z (of
-// a prefill) sees n_ctx + z positions; its q and scores are z q_st and
-// z sc_st floats on.
-template <int E>
-__global__ __launch_bounds__(OPS_TPB) void attn_scores_kernel(float *__restrict__ scores, const float *__restrict__ q,
-                                                              const float *__restrict__ kc, int n_ctx, int n_head_kv,
-                                                              int group, size_t q_st, size_t sc_st) {
-    constexpr int HD = 64 * E;
-    __shared__ float qs[kAttnMaxGroup * HD];
-    n_ctx += (int)blockIdx.z;
-    if (blockIdx.x * kScoresPPB >= (unsigned)n_ctx) return;  // the whole workgroup: past this query's positions
-    q += blockIdx.z * q_st;
-    scores += blockIdx.z * sc_st;
-    const int kv = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int t = threadIdx.x; t < group * HD; t += OPS_TPB) qs[t] = q[(size_t)kv * group * HD + t];
-    __syncthreads();
-    const size_t kv_len = (size_t)n_head_kv * HD;
-    // the wave's positions p0 + 4t: every K row is loaded before the dots
-    constexpr int PW = kScoresPPB / (OPS_TPB / 64);
-    const int p0 = blockIdx.x * kScoresPPB + w;
-    float kx[PW][E];
-#pragma unroll
-    for (int t = 0; t < PW; t++) {
-        const int p = min(p0 + t * (OPS_TPB / 64), n_ctx - 1);
-        const float *kr = kc + (size_t)p * kv_len + (size_t)kv * HD + lane * E;
-#pragma unroll
-        for (int e = 0; e < E; e++) kx[t][e] = kr[e];
-    }
-#pragma unroll
-    for (int t = 0; t < PW; t++) {
-        const int p = p0 + t * (OPS_TPB / 64);
-        if (p >= n_ctx) break;  // wave-uniform
-        for (int g = 0; g < group; g++) {
-            double d[E];
-#pragma unroll
-            for (int e = 0; e < E; e++) d[e] = (double)qs[g * HD + lane * E + e] * (double)kx[t][e];
-            const double sc = wave_pairwise<E>(d);
-            if (lane == 0) scores[(size_t)(kv * group + g) * n_ctx + p] = (float)sc;
-        }
-    }
-}
-
-// The pairwise tree (kernels.rs:21-42) of the N products x_i * y_i (exact
-// in f64), i in [B, B + N), N a power of two: both halves, then their sum,
-// the reference's adjacent-pair levels (it carries no odd tail at a power
-// of two). x a broadcast row in LDS, y the lane's row in LDS.
-template <int N, int B>
-__device__ __forceinline__ double tree_dot(const float *__restrict__ x, const float *__restrict__ y) {
-    if constexpr (N == 1)
-        return (double)x[B] * (double)y[B];
-    else if constexpr (N == 2)  // x1 y1 + x0 y0, both exact, rounded once: one fma
-        return fma((double)x[B + 1], (double)y[B + 1], (double)x[B] * (double)y[B]);
-    else
-        return tree_dot<N / 2, B>(x, y) + tree_dot<N / 2, B + N / 2>(x, y);
-}
-
-// Scores of a prefill chunk with one lane per position: the workgroup holds
-// the K rows of 64 positions (one kv head) in LDS and the q rows of up to qb
-// queries of the group's heads (at most 80 KB in all, so two workgroups
-// share a CU); wave w takes the (query, head)
-// pairs w, w + 4, ..., and each lane forms its position's whole dot as the
-// pairwise tree, with no exchange between lanes. Query z0 + zz sees n_ctx +
-// z0 + zz positions (causal). Each dot is the same tree of the same exact
-// products as attn_scores_kernel's, so the same bits; the lane butterflies
-// that bound that kernel are gone.
-constexpr int kLaneScoresPos = 64;
-template <int HD>
-__global__ __launch_bounds__(OPS_TPB) void attn_scores_lane_kernel(float *__restrict__ scores,
-                                                                   const float *__restrict__ q,
-                                                                   const float *__restrict__ kc, int n_ctx,
-                                                                   int n_head_kv, int group, size_t q_st,
-                                                                   size_t sc_st, int rows, int qb) {
-    constexpr int KP = HD + 1;  // K row pitch in floats: an odd pitch, no bank conflicts
-    extern __shared__ __align__(16) float qd[];  // [qb * group][HD], then K [64][KP]
-    const int p0 = blockIdx.x * kLaneScoresPos, kv = blockIdx.y, z0 = blockIdx.z * qb;
-    const int nz = min(qb, rows - z0), n_hi = n_ctx + z0 + nz - 1;  // positions of the block's last query
-    if (p0 >= n_hi) return;  // the whole workgroup
-    float *ks = qd + (size_t)qb * group * HD;
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int gh = group * HD;
-    const size_t kv_len = (size_t)n_head_kv * HD;
-    for (int idx = tid; idx < kLaneScoresPos * (HD / 4); idx += OPS_TPB) {
-        const int r = idx / (HD / 4), c4 = idx - r * (HD / 4);
-        const int p = min(p0 + r, n_hi - 1);
-        const float4 v = *(const float4 *)(kc + (size_t)p * kv_len + (size_t)kv * HD + 4 * c4);
-        float *d = ks + r * KP + 4 * c4;
-        d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
-    }
-    for (int idx = tid; idx < nz * gh; idx += OPS_TPB) {
-        const int zz = idx / gh, rr = idx - zz * gh;
-        qd[idx] = q[(size_t)(z0 + zz) * q_st + (size_t)kv * gh + rr];
-    }
-    __syncthreads();
-    const int p = p0 + lane;
-    const float *kr = ks + lane * KP;
-    for (int pair = wv; pair < nz * group; pair += OPS_TPB / 64) {
-        const int zz = pair / group, g = pair - zz * group;
-        const int nzc = n_ctx + z0 + zz;
-        if (p0 >= nzc) continue;  // no position of the tile for this query (wave-uniform)
-        const double sc = tree_dot<HD, 0>(qd + (size_t)pair * HD, kr);
-        if (p < nzc) scores[(size_t)(z0 + zz) * sc_st + (size_t)(kv * group + g) * nzc + p] = (float)sc;
-    }
-}
-
-// out[h][i] = (f32) of the sequential f64 sum over p of soft[h][p] * V[p][i]
-// (every product exact in f64). Lane = column i, the waves split p; the
-// partial sums S and absolute sums A meet in LDS. Any summation order of
-// n terms lies within gamma_n * A of the exact sum, so the sequential sum
-// lies in [S - e, S + e], e = (n + 66) 2^-52 A (with room for the rounding
-// of e and S +- e); when both ends round to the same f32 (same bits) that
-// is the reference's value, else the lane replays the sequential loop.
-constexpr int kPvBatch = 16;  // positions whose V loads a wave issues before summing
-constexpr int kPvCoop = 4;    // at most this many replays per wave run one column at a time
-constexpr int kPvChunk = 8;   // positions per lane loaded at once in such a replay
-template <int G>
-constexpr int pv_waves() { return G <= 4 ? 16 : 8; }  // the LDS partials stay within 64 KB
-// G: q heads per kv head, compile-time so that a batch's loads issue back to
-// back. Query z = blockIdx.z (of a prefill) sees n_ctx + z positions; its
-// soft, out, gz and gated rows are z times the strides in st on.
-struct PvStrides {
-    size_t soft, out, gz, gated;
-};
-template <int G>
-__global__ __launch_bounds__(pv_waves<G>() * 64) void attn_pv_kernel(float *__restrict__ out,
-                                                                    const float *__restrict__ soft,
-                                                                    const float *__restrict__ vc, int n_ctx,
-                                                                    int n_head_kv, int hd,
-                                                                    const float *__restrict__ gz, int gzs,
-                                                                    float *__restrict__ gated, PvStrides zs) {
-    constexpr int group = G, kPvWaves = pv_waves<G>();
-    __shared__ double part[2][kPvWaves][G][64];
-    n_ctx += (int)blockIdx.z;
-    soft += blockIdx.z * zs.soft;
-    out += blockIdx.z * zs.out;
-    if (gated) {
-        gz += blockIdx.z * zs.gz;
-        gated += blockIdx.z * zs.gated;
-    }
-    const int kv = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = blockIdx.x * 64 + lane;
-    const size_t kv_len = (size_t)n_head_kv * hd;
-    const float *vcol = vc + (size_t)kv * hd + i;
-    const float *sr = soft + (size_t)kv * group * n_ctx;
-    double S[G], A[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) S[g] = A[g] = 0.0;
-    // positions in batches of kPvBatch per wave, loads first (the sums only
-    // need some order: the bound below covers any)
-    for (int p0 = w; p0 < n_ctx; p0 += kPvWaves * kPvBatch) {
-        float vb[kPvBatch], sb[kPvBatch][G];
-#pragma unroll
-        for (int u = 0; u < kPvBatch; u++) {
-            const int p = min(p0 + u * kPvWaves, n_ctx - 1);
-            vb[u] = vcol[(size_t)p * kv_len];
-#pragma unroll
-            for (int g = 0; g < G; g++) sb[u][g] = sr[(size_t)g * n_ctx + p];
-        }
-#pragma unroll
-        for (int u = 0; u < kPvBatch; u++) {
-            const bool in = p0 + u * kPvWaves < n_ctx;
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                const double t = in ? (double)sb[u][g] * (double)vb[u] : 0.0;
-                S[g] += t;
-                A[g] += fabs(t);
-            }
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        part[0][w][g][lane] = S[g];
-        part[1][w][g][lane] = A[g];
-    }
-    __syncthreads();
-    double st = 0.0, at = 0.0;
-    if (w < group)
-        for (int u = 0; u < kPvWaves; u++) {
-            st += part[0][u][w][lane];
-            at += part[1][u][w][lane];
-        }
-    __syncthreads();  // part is free: a replay below uses it as its wave's scratch
-    if (w < group) {
-        const int g = w;
-        const double e = (double)(n_ctx + 66) * 0x1p-52 * at;
-        const float lo = (float)(st - e), hi = (float)(st + e);
-        float r = lo;
-        // the reference's sequential sum where the bound cannot decide
-        // (about 1e-4 of the outputs)
-        const bool need = __float_as_uint(lo) != __float_as_uint(hi);
-        unsigned long long mask = __ballot(need);
-        if (__popcll(mask) > kPvCoop) {
-            // many columns: each lane replays its own, loads in batches, the adds in order
-            if (need) {
-                constexpr int RB = 32;
-                double q = 0.0;
-                for (int p0 = 0; p0 < n_ctx; p0 += RB) {
-                    float vb[RB], sb[RB];
-#pragma unroll
-                    for (int u = 0; u < RB; u++) {
-                        const int p = min(p0 + u, n_ctx - 1);
-                        vb[u] = vcol[(size_t)p * kv_len];
-                        sb[u] = sr[(size_t)g * n_ctx + p];
-                    }
-#pragma unroll
-                    for (int u = 0; u < RB; u++)
-                        if (p0 + u < n_ctx) q += (double)sb[u] * (double)vb[u];
-                }
-                r = (float)q;
-            }
-        } else {
-            // a few columns: the wave replays them one at a time, every lane
-            // forming the products of its positions (loads in parallel) into
-            // the wave's LDS scratch, then all lanes adding them in position
-            // order (broadcast reads; the same sum in each lane)
-            double *buf = &part[0][0][0][0] + (size_t)w * 64 * kPvChunk;  // within part: kPvWaves >= 4
-            while (mask) {
-                const int l = __ffsll(mask) - 1;
-                mask &= mask - 1;
-                const float *vl = vc + (size_t)kv * hd + blockIdx.x * 64 + l;
-                double q = 0.0;
-                for (int p0 = 0; p0 < n_ctx; p0 += 64 * kPvChunk) {
-#pragma unroll
-                    for (int k = 0; k < kPvChunk; k++) {
-                        const int p = min(p0 + 64 * k + lane, n_ctx - 1);
-                        buf[64 * k + lane] = (double)sr[(size_t)g * n_ctx + p] * (double)vl[(size_t)p * kv_len];
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    const int m = min(64 * kPvChunk, n_ctx - p0);
-                    // the reads of the next 8 values issue before the adds of these 8
-                    int p = 0;
-                    double b[8];
-                    if (m >= 8) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) b[u] = buf[u];
-                    }
-                    for (; p + 8 <= m; p += 8) {
-                        double nb[8];
-                        const int pn = p + 16 <= m ? p + 8 : p;  // the last batch rereads itself
-#pragma unroll
-                        for (int u = 0; u < 8; u++) nb[u] = buf[pn + u];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) q += b[u];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) b[u] = nb[u];
-                    }
-                    for (; p < m; p++) q += buf[p];
-                    // every lane's reads are done before the next chunk's writes
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-                if (lane == l) r = (float)q;
-            }
-        }
-        out[(size_t)(kv * group + g) * hd + i] = r;
-        // the gated output (qwen35_forward.rs:677-684, as mul_act_kernel)
-        if (gated) gated[(size_t)(kv * group + g) * hd + i] = __fmul_rn(r, sigmoid1(gz[(size_t)(kv * group + g) * gzs + i]));
-    }
-}
-
-// attn_pv_kernel for a prefill chunk: a workgroup takes the NP = (16 / G) *
-// G (query, head) pairs of QB = 16 / G consecutive queries and the G heads
-// of kv head blockIdx.y, lane = column blockIdx.x * 64 + lane, so each V
-// load serves all NP pairs. Wave w takes the 16-position batches w, w + 4,
-// ...; a pair's soft values of a batch are uniform (scalar) loads. Each
-// product is exact in f64, so S += s * v and A += |s * v| are single fused
-// multiply-adds with the values of the separate multiply and add. The four
-// waves' S and A meet in LDS, then the bound decides each output as in
-// attn_pv_kernel, or the lane replays the sequential sum.
-constexpr int kPvRowsWaves = 4, kPvRowsBatch = 16;
-template <int G>
-__global__ __launch_bounds__(kPvRowsWaves * 64) void attn_pv_rows_kernel(
-    float *__restrict__ out, const float *__restrict__ soft, const float *__restrict__ vc, int n_ctx, int n_head_kv,
-    int hd, int rows, const float *__restrict__ gz, int gzs, float *__restrict__ gated, PvStrides zs) {
-    constexpr int QB = 16 / G, NP = QB * G;
-    __shared__ double part[kPvRowsWaves][NP][64];
-    static_assert(NP >= kPvChunk, "a wave's part rows hold its replay chunk");
-    const int kv = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int z0 = blockIdx.z * QB, nz = min(QB, rows - z0);
-    const int i = blockIdx.x * 64 + lane;
-    const size_t kv_len = (size_t)n_head_kv * hd;
-    const float *vcol = vc + (size_t)kv * hd + i;
-    const int n_hi = n_ctx + z0 + nz - 1;  // positions of the block's last query
-    // soft row of pair q: query z0 + q / G, head kv * G + q % G
-    auto srow = [&](int q) {
-        const int zz = q / G, nzc = n_ctx + z0 + zz;
-        return soft + (size_t)(z0 + zz) * zs.soft + (size_t)(kv * G + q % G) * nzc;
-    };
-    double S[NP], A[NP];
-#pragma unroll
-    for (int q = 0; q < NP; q++) S[q] = A[q] = 0.0;
-    for (int pb = w * kPvRowsBatch; pb < n_hi; pb += kPvRowsWaves * kPvRowsBatch) {
-        double vd[kPvRowsBatch];
-#pragma unroll
-        for (int u = 0; u < kPvRowsBatch; u++) vd[u] = (double)vcol[(size_t)min(pb + u, n_hi - 1) * kv_len];
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            const int zz = q / G, nzc = n_ctx + z0 + zz;
-            if (zz >= nz || pb >= nzc) continue;  // wave-uniform
-            const float *sr = srow(q) + pb;
-            if (pb + kPvRowsBatch <= nzc) {
-#pragma unroll
-                for (int u = 0; u < kPvRowsBatch; u++) {
-                    const double sv = (double)sr[u];
-                    S[q] = fma(sv, vd[u], S[q]);
-                    A[q] = fma(fabs(sv), fabs(vd[u]), A[q]);
-                }
-            } else {
-                const int m = nzc - pb;
-#pragma unroll
-                for (int u = 0; u < kPvRowsBatch; u++)
-                    if (u < m) {
-                        const double sv = (double)sr[u];
-                        S[q] = fma(sv, vd[u], S[q]);
-                        A[q] = fma(fabs(sv), fabs(vd[u]), A[q]);
-                    }
-            }
-        }
-    }
-    // the waves' partials: S, then A, through the one LDS array
-    double st[(NP + kPvRowsWaves - 1) / kPvRowsWaves], at[(NP + kPvRowsWaves - 1) / kPvRowsWaves];
-#pragma unroll
-    for (int ph = 0; ph < 2; ph++) {
-#pragma unroll
-        for (int q = 0; q < NP; q++) part[w][q][lane] = ph == 0 ? S[q] : A[q];
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < (NP + kPvRowsWaves - 1) / kPvRowsWaves; k++) {
-            const int q = w + kPvRowsWaves * k;
-            double t = 0.0;
-            if (q < NP)
-#pragma unroll
-                for (int u = 0; u < kPvRowsWaves; u++) t += part[u][q][lane];
-            (ph == 0 ? st : at)[k] = t;
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < (NP + kPvRowsWaves - 1) / kPvRowsWaves; k++) {
-        const int q = w + kPvRowsWaves * k;
-        if (q >= NP) break;
-        const int zz = q / G, g = q % G, nzc = n_ctx + z0 + zz;
-        if (zz >= nz) break;  // wave-uniform; later k only higher zz
-        const double e = (double)(nzc + 66) * 0x1p-52 * at[k];
-        const float lo = (float)(st[k] - e), hi = (float)(st[k] + e);
-        float r = lo;
-        // the reference's sequential sum where the bound cannot decide
-        const bool need = __float_as_uint(lo) != __float_as_uint(hi);
-        unsigned long long mask = __ballot(need);
-        const float *sr = srow(q);
-        if (__popcll(mask) > kPvCoop) {
-            // many columns: each lane replays its own
-            if (need) {
-                double qs = 0.0;
-                for (int p0 = 0; p0 < nzc; p0 += 16) {
-                    float vb[16], sb[16];
-#pragma unroll
-                    for (int u = 0; u < 16; u++) {
-                        const int p = min(p0 + u, nzc - 1);
-                        vb[u] = vcol[(size_t)p * kv_len];
-                        sb[u] = sr[p];
-                    }
-#pragma unroll
-                    for (int u = 0; u < 16; u++)
-                        if (p0 + u < nzc) qs += (double)sb[u] * (double)vb[u];
-                }
-                r = (float)qs;
-            }
-        } else {
-            // a few columns, one at a time: every lane forms the products of
-            // its positions (loads in parallel) into the wave's LDS scratch
-            // (part is free after the reductions), then all lanes add them in
-            // position order (broadcast reads; the same sum in each lane)
-            double *buf = &part[w][0][0];
-            while (mask) {
-                const int l = __ffsll(mask) - 1;
-                mask &= mask - 1;
-                const float *vl = vc + (size_t)kv * hd + blockIdx.x * 64 + l;
-                double qs = 0.0;
-                for (int p0 = 0; p0 < nzc; p0 += 64 * kPvChunk) {
-#pragma unroll
-                    for (int c = 0; c < kPvChunk; c++) {
-                        const int p = min(p0 + 64 * c + lane, nzc - 1);
-                        buf[64 * c + lane] = (double)sr[p] * (double)vl[(size_t)p * kv_len];
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    const int m = min(64 * kPvChunk, nzc - p0);
-                    // the reads of the next eight values issue before the adds of these eight
-                    int p = 0;
-                    double bb[8];
-                    if (m >= 8) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) bb[u] = buf[u];
-                    }
-                    for (; p + 8 <= m; p += 8) {
-                        double nb[8];
-                        const int pn = p + 16 <= m ? p + 8 : p;  // the last group rereads itself
-#pragma unroll
-                        for (int u = 0; u < 8; u++) nb[u] = buf[pn + u];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) qs += bb[u];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) bb[u] = nb[u];
-                    }
-                    for (; p < m; p++) qs += buf[p];
-                    // every lane's reads are done before the next chunk's writes
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-                if (lane == l) r = (float)qs;
-            }
-        }
-        float *o = out + (size_t)(z0 + zz) * zs.out;
-        o[(size_t)(kv * G + g) * hd + i] = r;
-        if (gated)
-            gated[(size_t)(z0 + zz) * zs.gated + (size_t)(kv * G + g) * hd + i] =
-                __fmul_rn(r, sigmoid1(gz[(size_t)(z0 + zz) * zs.gz + (size_t)(kv * G + g) * gzs + i]));
-    }
-}
-
 // ---- glue of the layer forward (qwen35_forward.rs:333-710) ----------------
 // GatedDeltaNet gates (:405-419): beta = sigmoid(beta_raw), sp =
 // softplus(alpha + dt_bias), gate = sp * a, per v head.
@@ -1373,19 +807,6 @@ hipError_t launch_l2norm(float *data, int dim, int rows, float eps, hipStream_t 
     return hipGetLastError();
 }
 
-int softmax_max_len() { return kSmChunk * kSmMaxChunks; }
-
-hipError_t launch_softmax(float *out, const float *x, int n, int rows, float scale, hipStream_t s) {
-    if (rows == 0 || n == 0) return hipSuccess;
-    if (n > softmax_max_len()) return hipErrorInvalidValue;
-    if (n <= kSmWaveMax)
-        hipLaunchKernelGGL(softmax_wave_kernel, dim3((rows + OPS_TPB / 64 - 1) / (OPS_TPB / 64)), dim3(OPS_TPB), 0, s,
-                           out, x, n, scale, 0, (size_t)0, rows);
-    else
-        hipLaunchKernelGGL(softmax_kernel, dim3(rows), dim3(OPS_TPB), 0, s, out, x, n, scale, 0, (size_t)0);
-    return hipGetLastError();
-}
-
 hipError_t launch_unary(int op, const float *x, size_t n, float *out, hipStream_t s) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(unary_kernel, dim3(ops_grid(n)), dim3(OPS_TPB), 0, s, op, x, n, out);
@@ -1458,95 +879,6 @@ hipError_t launch_rope_imrope(float *x, int rows, int n, int n_rot, double theta
     hipLaunchKernelGGL(rope_imrope_kernel, dim3(ops_grid((size_t)rows * nrot3)), dim3(OPS_TPB), 0, s, x, rows, n,
                        n_rot, theta_scale, (double)pos);
     return hipGetLastError();
-}
-
-bool attn_shape_ok(int hd, int group) {
-    return (hd == 64 || hd == 128 || hd == 256 || hd == 512) && group >= 1 && group <= kAttnMaxGroup;
-}
-
-hipError_t launch_attn_rows(float *out, size_t out_st, float *soft, size_t soft_st, const float *q, size_t q_st,
-                            const float *kc, const float *vc, int n_ctx, int rows, int n_head_kv, int hd, int group,
-                            float kq_scale, hipStream_t s, const float *gz, int gzs, size_t gz_st, float *gated,
-                            size_t gated_st) {
-    if (n_ctx <= 0 || n_head_kv <= 0 || rows <= 0) return hipSuccess;
-    const int n_last = n_ctx + rows - 1;
-    if (!attn_shape_ok(hd, group) || n_last > softmax_max_len() || rows > 65535) return hipErrorInvalidValue;
-    if (rows > 1 && hd <= 256) {
-        // a prefill chunk: lane-per-position dots, blocks of qb queries whose
-        // q rows and the 64 K rows fit 80 KB of LDS
-        const size_t kbytes = (size_t)kLaneScoresPos * (hd + 1) * 4;
-        const int qb = (int)std::max<size_t>(1, std::min<size_t>(8, (80 * 1024 - kbytes) / ((size_t)group * hd * 4)));
-        const size_t lds = (size_t)qb * group * hd * 4 + kbytes;
-        const dim3 gl((n_last + kLaneScoresPos - 1) / kLaneScoresPos, n_head_kv, (rows + qb - 1) / qb);
-        hipError_t e = hipSuccess;
-        auto go = [&](const void *k, auto launch) {
-            if ((e = allow_lds(k, lds)) == hipSuccess) launch();
-        };
-        switch (hd) {
-            case 64: go((const void *)attn_scores_lane_kernel<64>, [&] { hipLaunchKernelGGL(attn_scores_lane_kernel<64>, gl, dim3(OPS_TPB), lds, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st, rows, qb); }); break;
-            case 128: go((const void *)attn_scores_lane_kernel<128>, [&] { hipLaunchKernelGGL(attn_scores_lane_kernel<128>, gl, dim3(OPS_TPB), lds, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st, rows, qb); }); break;
-            default: go((const void *)attn_scores_lane_kernel<256>, [&] { hipLaunchKernelGGL(attn_scores_lane_kernel<256>, gl, dim3(OPS_TPB), lds, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st, rows, qb); }); break;
-        }
-        if (e != hipSuccess) return e;
-    } else {
-        const dim3 gs((n_last + kScoresPPB - 1) / kScoresPPB, n_head_kv, rows);
-        switch (hd) {
-            case 64: hipLaunchKernelGGL(attn_scores_kernel<1>, gs, dim3(OPS_TPB), 0, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st); break;
-            case 128: hipLaunchKernelGGL(attn_scores_kernel<2>, gs, dim3(OPS_TPB), 0, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st); break;
-            case 256: hipLaunchKernelGGL(attn_scores_kernel<4>, gs, dim3(OPS_TPB), 0, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st); break;
-            default: hipLaunchKernelGGL(attn_scores_kernel<8>, gs, dim3(OPS_TPB), 0, s, soft, q, kc, n_ctx, n_head_kv, group, q_st, soft_st); break;
-        }
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (n_last <= kSmWaveMax)
-        hipLaunchKernelGGL(softmax_wave_kernel, dim3((n_head_kv * group + OPS_TPB / 64 - 1) / (OPS_TPB / 64), rows),
-                           dim3(OPS_TPB), 0, s, soft, soft, n_ctx, kq_scale, 1, soft_st, n_head_kv * group);
-    else
-        hipLaunchKernelGGL(softmax_kernel, dim3(n_head_kv * group, rows), dim3(OPS_TPB), 0, s, soft, soft, n_ctx,
-                           kq_scale, 1, soft_st);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    const PvStrides pst{soft_st, out_st, gz_st, gated_st};
-    if (rows > 1) {
-        // a prefill chunk: 16 / group queries per workgroup
-#define UQ_PVR(G) hipLaunchKernelGGL(attn_pv_rows_kernel<G>, dim3(hd / 64, n_head_kv, (rows + 16 / G - 1) / (16 / G)), \
-                                     dim3(kPvRowsWaves * 64), 0, s, out, soft, vc, n_ctx, n_head_kv, hd, rows, gz, gzs, \
-                                     gated, pst)
-        switch (group) {
-            case 1: UQ_PVR(1); break;
-            case 2: UQ_PVR(2); break;
-            case 3: UQ_PVR(3); break;
-            case 4: UQ_PVR(4); break;
-            case 5: UQ_PVR(5); break;
-            case 6: UQ_PVR(6); break;
-            case 7: UQ_PVR(7); break;
-            default: UQ_PVR(8); break;
-        }
-#undef UQ_PVR
-        return hipGetLastError();
-    }
-    const dim3 gp(hd / 64, n_head_kv, rows);
-#define UQ_PV(G) hipLaunchKernelGGL(attn_pv_kernel<G>, gp, dim3(pv_waves<G>() * 64), 0, s, out, soft, vc, n_ctx, \
-                                    n_head_kv, hd, gz, gzs, gated, pst)
-    switch (group) {
-        case 1: UQ_PV(1); break;
-        case 2: UQ_PV(2); break;
-        case 3: UQ_PV(3); break;
-        case 4: UQ_PV(4); break;
-        case 5: UQ_PV(5); break;
-        case 6: UQ_PV(6); break;
-        case 7: UQ_PV(7); break;
-        default: UQ_PV(8); break;
-    }
-#undef UQ_PV
-    return hipGetLastError();
-}
-
-hipError_t launch_attn_decode(float *out, float *soft, const float *q, const float *kc, const float *vc, int n_ctx,
-                              int n_head_kv, int hd, int group, float kq_scale, hipStream_t s, const float *gz,
-                              int gzs, float *gated) {
-    return launch_attn_rows(out, 0, soft, 0, q, 0, kc, vc, n_ctx, 1, n_head_kv, hd, group, kq_scale, s, gz, gzs, 0,
-                            gated, 0);
 }
 
 hipError_t launch_gdn_gates(const float *beta_raw, const float *alpha, const float *dt_bias, const float *a,
