@@ -110,6 +110,20 @@ def test_gemm_q8k_shapes(dtype, K, N, M):
 
 
 @pytest.mark.parametrize("dtype", [S.Q4_K, S.Q6_K])
+@pytest.mark.parametrize("M,N", [(61, 500), (99, 2040), (250, 2040), (509, 2040), (509, 4090)])
+def test_gemm_q8k_shape_of_least_time(dtype, M, N):
+    """Nine blocks at row counts and widths (ragged both ways) where the
+    estimate picks, in this order, the K-parallel kernel, four waves of 16
+    rows, of 32, eight of 32 (Q4_K; four for Q6_K) and eight of 64."""
+    K = 9 * 256
+    w = S.weights(dtype, N, K, seed=N + M + dtype)
+    X = S.activations(K, seed=M * 5 + dtype, rows=M).reshape(M, K)
+    Y = run(dtype, w, K, N, X)
+    rows = sorted({0, 15, 16, 31, 32, 33, M // 2, M - 2, M - 1})
+    assert_rows(Y, oracle_rows(dtype, w, K, N, X, rows), f"gemm_q8k M={M} N={N}")
+
+
+@pytest.mark.parametrize("dtype", [S.Q4_K, S.Q6_K])
 def test_gemm_q8k_equals_per_row_gemv_q8k(dtype):
     """Every row equals the device's own gemv_quant_q8k of that row (the
     decode kernel, checked against the oracle elsewhere), at a shape with

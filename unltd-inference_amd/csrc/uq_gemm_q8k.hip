@@ -678,41 +678,55 @@ hipError_t q8k_kpar_launch(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s)
     return hipGetLastError();
 }
 
-// Rows per wave (and workgroup): 16 for M <= 16; 64 for M > 128 while the
-// 64 x 128 workgroup tiles number at least one per CU (eight waves, two per
-// SIMD: the B operands decoded once for 64 rows); 32 while 32 x 64 tiles
-// (four 16-column waves) number at least one per CU; else 16. Waves
-// (16-column tiles) per workgroup: four while the workgroups number at
-// least one per CU, else two while they do, else one. Four waves hold a
-// two-slot ring small enough for three workgroups per CU, where six waves'
-// held two. Measured over the prefill's projections (a sweep of every
-// wave count and tile height): at M = 128 the rule is the best shape or
-// within a few percent of it, e.g. Q4_K 8192 x 4096 35 us (six waves: 54),
-// Q6_K 4096 x 12288 75 us (16-row tiles: 96); at M = 512 the 64-row tiles
-// stay best for N >= 4096 (Q4_K 12288 x 4096 144 against 155 on 32-row
-// ones) and N = 1024 takes 32-row tiles (34 against 47 us).
-template <bool Q6, int RT>
-hipError_t q8k_width(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s) {
-    const int cus = 256, ntm = (M + 16 * RT - 1) / (16 * RT);
-    if (ntm * j.cols(64) >= cus) return q8k_launch<Q6, 4, RT>(j, M, ws, s);
-    if (ntm * j.cols(32) >= cus) return q8k_launch<Q6, 2, RT>(j, M, ws, s);
-    return q8k_launch<Q6, 1, RT>(j, M, ws, s);
-}
-// The rule counts column tiles over all the launch's segments.
+// Which shape a launch takes: the least estimated time of these five. A CU
+// walks its share of the workgroups, ceil(G / 256) of the G, as many at a time
+// as its LDS and registers hold, each over K / 256 blocks in lockstep, so the
+// time is the blocks times a cost per block that depends on how many share the
+// CU (more of them hide each other's latency, at less than their number's
+// cost). The costs (us per block with 1, 2, 3 workgroups on a CU) are a least-
+// squares fit over a sweep of every shape at 17 row counts from 8 to 512 and
+// six K x N from 2048 x 700 to 12288 x 4096; the estimate is within 5% of the
+// sweep's times (standard deviation), its choice within 1.3% (Q4_K) and 0.7%
+// (Q6_K) of the best shape's in the geometric mean, where one workgroup per CU
+// as the threshold between shapes was 9% and 12% off. Examples (K x N):
+// Q6_K 12288 x 4096 at M = 77 86 -> 68 us, at 400 218 -> 153, 4096 x 12288 at
+// 160 109 -> 73, Q4_K 4096 x 12288 at 160 86 -> 53.
+struct Q8Shape {
+    int nw, rt;       // 16-column waves, 16-row tiles; rt 0: the K-parallel kernel, four waves per 16 x 16 tile
+    int held[2];      // workgroups a CU holds, [Q6_K]
+    float cost[2][3];  // [Q6_K][workgroups on the CU - 1]
+};
+constexpr Q8Shape kQ8Shapes[] = {
+    {1, 0, {1, 1}, {{0.476f, 0, 0}, {0.512f, 0, 0}}},
+    {4, 1, {3, 3}, {{0.768f, 1.102f, 1.347f}, {0.981f, 1.555f, 2.074f}}},
+    {4, 2, {3, 2}, {{1.010f, 1.437f, 1.942f}, {1.214f, 1.920f, 0}}},
+    {8, 2, {1, 1}, {{1.410f, 0, 0}, {1.993f, 0, 0}}},
+    {8, 4, {1, 1}, {{2.270f, 0, 0}, {2.919f, 0, 0}}},
+};
 template <bool Q6>
 hipError_t q8k_shape(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s) {
-    const int cus = 256, K = j.K();
-    // 16-row tiles of 16 columns numbering at most one per CU, and K long
-    // enough to split (the 32-wide projections of a prefill, for one): the
-    // K-parallel kernel, four waves per tile
-    if (((M + 15) / 16) * j.cols(16) <= cus && K >= 8 * 256) return q8k_kpar_launch<Q6, 4>(j, M, ws, s);
-    // M <= 32 at long K (K > 8192: a 16- or 32-row wave would walk over 32
-    // blocks alone), up to two workgroups per CU: the K-parallel kernel
-    if (M <= 32 && ((M + 15) / 16) * j.cols(16) <= 2 * cus && K > 8192) return q8k_kpar_launch<Q6, 4>(j, M, ws, s);
-    if (M <= 16) return q8k_width<Q6, 1>(j, M, ws, s);
-    if (M > 128 && ((M + 63) / 64) * j.cols(128) >= cus) return q8k_launch<Q6, 8, 4>(j, M, ws, s);
-    if (((M + 31) / 32) * j.cols(64) >= cus) return q8k_width<Q6, 2>(j, M, ws, s);
-    return q8k_width<Q6, 1>(j, M, ws, s);
+    const int K = j.K();
+    int best = 1;
+    float least = 0.0f;
+    for (int i = 0; i < 5; i++) {
+        const Q8Shape &p = kQ8Shapes[i];
+        if (p.rt == 0 && K < 8 * 256) continue;  // four blocks at a time: at least two rounds
+        if (p.rt == 4 && M <= 128) continue;     // the planes' rows are padded to 32
+        if (Q6 && i == 3) continue;              // never the least for Q6_K
+        const int tm = 16 * (p.rt ? p.rt : 1), held = p.held[Q6];
+        const long groups = (long)((M + tm - 1) / tm) * j.cols(16 * p.nw), q = (groups + 255) / 256;
+        const float *c = p.cost[Q6];
+        const float t = (float)(q / held) * c[held - 1] + (q % held ? c[q % held - 1] : 0.0f);
+        if (least == 0.0f || t < least) least = t, best = i;
+    }
+    switch (best) {  // 3: Q4_K only
+        case 0: return q8k_kpar_launch<Q6, 4>(j, M, ws, s);
+        case 1: return q8k_launch<Q6, 4, 1>(j, M, ws, s);
+        case 2: return q8k_launch<Q6, 4, 2>(j, M, ws, s);
+        case 3:
+            if constexpr (!Q6) return q8k_launch<Q6, 8, 2>(j, M, ws, s);
+        default: return q8k_launch<Q6, 8, 4>(j, M, ws, s);
+    }
 }
 
 __global__ __launch_bounds__(256) void q8k_fill_zero_kernel(float *__restrict__ Y, size_t n) {
