@@ -133,6 +133,49 @@ __global__ __launch_bounds__(TPB) void rmsnorm_kernel(float *__restrict__ out, c
     }
 }
 
+// rmsnorm_kernel for many rows of n <= 128 (the gated norm of a prefill's head
+// outputs): a wave per row, two elements a lane, no LDS and no barrier; the
+// sum is the wave's tree with the bound of seq_sum_f32, or, undecided, the
+// sequential loop with each value taken from its lane by readlane. 16384 rows
+// of 128 with z in 9.2 us, 16.7 on a workgroup per row.
+constexpr int kNormRows = 4;  // rows (waves) per workgroup
+__global__ __launch_bounds__(64 * kNormRows) void rmsnorm_wave_kernel(float *__restrict__ out, const float *__restrict__ x,
+                                                                      const float *__restrict__ w, int n, float eps,
+                                                                      int xs, int ys, const float *__restrict__ z,
+                                                                      int rows) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * kNormRows + (int)(threadIdx.x >> 6);
+    if (row >= rows) return;  // the whole wave
+    const float *xr = x + (size_t)row * xs;
+    float v[2], wv[2], zv[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int i = lane + 64 * k;
+        v[k] = i < n ? xr[i] : 0.0f;
+        wv[k] = i < n ? w[i] : 0.0f;
+        zv[k] = z && i < n ? z[(size_t)row * ys + i] : 0.0f;
+    }
+    const double S = wave_sum_d((double)__fmul_rn(v[0], v[0]) + (double)__fmul_rn(v[1], v[1]));
+    const double dn = (double)n, e = (double)(n + 66) * 0x1p-52 * S;
+    float mean = (float)((S - e) / dn);
+    if (__float_as_uint(mean) != __float_as_uint((float)((S + e) / dn))) {  // wave-uniform; -0 and +0 replay too
+        double q = 0.0;
+        for (int i = 0; i < n; i++) {
+            const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(i < 64 ? v[0] : v[1]), i & 63));
+            q += (double)__fmul_rn(t, t);
+        }
+        mean = (float)(q / dn);
+    }
+    const float scale = __fdiv_rn(1.0f, sqrtf_cr(__fadd_rn(mean, eps)));
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int i = lane + 64 * k;
+        if (i >= n) break;
+        float y = __fmul_rn(__fmul_rn(v[k], scale), wv[k]);
+        if (z) y = __fmul_rn(y, silu1(zv[k]));
+        out[(size_t)row * ys + i] = y;
+    }
+}
+
 // l2_norm_rows (kernels.rs:236-256), in place, one workgroup per row.
 __global__ __launch_bounds__(OPS_TPB) void l2norm_kernel(float *__restrict__ data, int dim, float eps) {
     __shared__ double red[OPS_TPB / 64];
@@ -317,71 +360,88 @@ __global__ __launch_bounds__(64 * kGdnWaves) void gdn_step_wg_kernel(float *__re
 // independent per token and run as row-parallel launches around the scan.
 
 // Conv, silu and l2 norm of nt tokens (gdn_conv_norm_kernel per token),
-// one wave per unit (b, t), four units a workgroup: for b < n_chunks the
-// wave forms chunk b of token t into cv[t] (the q and k chunks normalised),
-// lane l its channels l and l + 64 (hd <= 128); the window seen by token t
+// one wave per chunk b and four consecutive tokens, four chunks a workgroup:
+// for b < n_chunks the wave forms chunk b of its tokens t into cv[t] (the q
+// and k chunks normalised), lane l its channels l and l + 64 (hd <= 128); the
+// taps are loaded once and each row once for the four tokens (512 tokens of
+// 8192 channels in 15.9 us, 24.4 with a token a wave); the window seen by token t
 // is entries t .. t + d_conv - 1 of the sequence [win rows 0 .. d_conv - 2;
 // qkv rows 0 .. nt - 1]. The norm's sum of squares is the wave's tree with
 // the bound of seq_sum_f32, or, undecided, the sequential loop with each
-// value taken from its lane by readlane. Unit (n_chunks, t) forms token t's
+// value taken from its lane by readlane. Chunk n_chunks forms the tokens'
 // gates per v head in place: beta_raw becomes beta = sigmoid(beta_raw),
 // alpha becomes exp(gate), gate = softplus(alpha + dt_bias) * a
 // (gdn_gates_kernel, then the step's exp of the gate).
-constexpr int kConvUnits = 4;  // units (waves) per workgroup
+constexpr int kConvUnits = 4;   // units (waves) per workgroup
+constexpr int kConvTokens = 4;  // consecutive tokens of a wave: its taps loaded once, a row once for all the tokens it is in
+template <int CK>  // d_conv, 0: any up to 9
 __global__ __launch_bounds__(64 * kConvUnits) void gdn_conv_norm_rows_kernel(
     const float *__restrict__ win, const float *__restrict__ kern, const float *__restrict__ qkv,
-    float *__restrict__ cv, int d_conv, int channels, int hd, int n_qk, float eps, float *__restrict__ beta,
-    float *__restrict__ gexp, const float *__restrict__ dt_bias, const float *__restrict__ a, int n_v) {
-    const int lane = threadIdx.x & 63, t = blockIdx.y, n_chunks = channels / hd;
-    const int b = blockIdx.x * kConvUnits + (int)(threadIdx.x >> 6);
+    float *__restrict__ cv, int dc, int channels, int hd, int n_qk, float eps, float *__restrict__ beta,
+    float *__restrict__ gexp, const float *__restrict__ dt_bias, const float *__restrict__ a, int n_v, int nt) {
+    constexpr int TAPS = CK ? CK : 9, ROWS = TAPS - 1 + kConvTokens;
+    const int d_conv = CK ? CK : dc;
+    const int lane = threadIdx.x & 63, t0 = blockIdx.y * kConvTokens, nn = min(kConvTokens, nt - t0);
+    const int n_chunks = channels / hd, b = blockIdx.x * kConvUnits + (int)(threadIdx.x >> 6);
     if (b > n_chunks) return;  // the whole wave
     if (b == n_chunks) {
-        for (int h = lane; h < n_v; h += 64) {
-            const size_t i = (size_t)t * n_v + h;
-            const float br = beta[i], al = gexp[i];
-            beta[i] = sigmoid1(br);
-            gexp[i] = expf_cr(__fmul_rn(softplus1(__fadd_rn(al, dt_bias[h])), a[h]));
+        for (int i = lane; i < nn * n_v; i += 64) {
+            const size_t o = (size_t)t0 * n_v + i;
+            const int h = i % n_v;
+            const float br = beta[o], al = gexp[o];
+            beta[o] = sigmoid1(br);
+            gexp[o] = expf_cr(__fmul_rn(softplus1(__fadd_rn(al, dt_bias[h])), a[h]));
         }
         return;
     }
     const bool norm = b < 2 * n_qk;  // wave-uniform
-    float v[2] = {0.0f, 0.0f};
-    double s = 0.0;
+    float v[kConvTokens][2];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const int j = lane + 64 * k;
-        if (j >= hd) break;
-        const int c = b * hd + j;
-        float x = 0.0f;
-        for (int tau = 0; tau < d_conv; tau++) {
-            const int u = t + tau;
-            const float xv = u < d_conv - 1 ? win[(size_t)u * channels + c] : qkv[(size_t)(u - d_conv + 1) * channels + c];
-            x = __fadd_rn(x, __fmul_rn(xv, kern[(size_t)c * d_conv + tau]));
-        }
-        v[k] = silu1(x);
-        if (norm)
-            s += (double)__fmul_rn(v[k], v[k]);
-        else
-            cv[(size_t)t * channels + c] = v[k];
-    }
-    if (!norm) return;
-    // l2_norm_rows of the chunk: (float) of the sequential f64 sum of squares
-    const double S = wave_sum_d(s);  // the same in every lane
-    const double e = (double)(hd + 66) * 0x1p-52 * S;
-    float sum32 = (float)(S - e);
-    if (__float_as_uint(sum32) != __float_as_uint((float)(S + e))) {  // wave-uniform; -0 and +0 replay too
-        double q = 0.0;
-        for (int i = 0; i < hd; i++) {
-            const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(i < 64 ? v[0] : v[1]), i & 63));
-            q += (double)__fmul_rn(x, x);
-        }
-        sum32 = (float)q;
-    }
-    const float scale = __fdiv_rn(1.0f, fmaxf(sqrtf_cr(sum32), eps));
+        const bool in = j < hd;
+        const int c = b * hd + (in ? j : 0);
+        float tap[TAPS], row[ROWS];
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int j = lane + 64 * k;
-        if (j < hd) cv[(size_t)t * channels + b * hd + j] = __fmul_rn(v[k], scale);
+        for (int tau = 0; tau < TAPS; tau++) tap[tau] = tau < d_conv ? kern[(size_t)c * d_conv + tau] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < ROWS; u++) {  // entries t0 .. t0 + d_conv + nn - 2 of the sequence
+            const int e = t0 + min(u, d_conv - 2 + nn);
+            row[u] = e < d_conv - 1 ? win[(size_t)e * channels + c] : qkv[(size_t)(e - d_conv + 1) * channels + c];
+        }
+#pragma unroll
+        for (int t = 0; t < kConvTokens; t++) {
+            float x = 0.0f;
+#pragma unroll
+            for (int tau = 0; tau < TAPS; tau++)
+                if (tau < d_conv) x = __fadd_rn(x, __fmul_rn(row[t + tau], tap[tau]));
+            v[t][k] = in ? silu1(x) : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < kConvTokens; t++) {
+        if (t >= nn) break;  // uniform
+        float scale = 1.0f;
+        if (norm) {
+            // l2_norm_rows of the chunk: (float) of the sequential f64 sum of squares
+            const double S = wave_sum_d((double)__fmul_rn(v[t][0], v[t][0]) + (double)__fmul_rn(v[t][1], v[t][1]));
+            const double e = (double)(hd + 66) * 0x1p-52 * S;  // S the same in every lane
+            float sum32 = (float)(S - e);
+            if (__float_as_uint(sum32) != __float_as_uint((float)(S + e))) {  // wave-uniform; -0 and +0 replay too
+                double q = 0.0;
+                for (int i = 0; i < hd; i++) {
+                    const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(i < 64 ? v[t][0] : v[t][1]), i & 63));
+                    q += (double)__fmul_rn(x, x);
+                }
+                sum32 = (float)q;
+            }
+            scale = __fdiv_rn(1.0f, fmaxf(sqrtf_cr(sum32), eps));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int j = lane + 64 * k;
+            if (j < hd) cv[(size_t)(t0 + t) * channels + b * hd + j] = norm ? __fmul_rn(v[t][k], scale) : v[t][k];
+        }
     }
 }
 
@@ -420,7 +480,9 @@ __device__ __forceinline__ void conv_window_channel(float *__restrict__ win, con
 // (twice the waves of sixteen, half the instructions each) measured 294 us
 // for 512 tokens of a 128-dim head as single-wave workgroups, which the
 // hardware doubled up on SIMDs, as sixteen rows per lane did (288 us), and
-// 226 us four to a workgroup.
+// 226-239 us four to a workgroup. One wave a SIMD: the instructions of a token
+// are the time. 206 us with the bound's sum in f32 and the decision mostly on
+// S's own bits (below).
 constexpr int kScanWaves = 4;
 template <int RB>
 __device__ __forceinline__ double col_sum_d(double v) {
@@ -428,6 +490,14 @@ __device__ __forceinline__ double col_sum_d(double v) {
     v += dpp_d<0x4E>(v);
     if constexpr (RB >= 8) v += dpp_d<0x141>(v);
     if constexpr (RB == 16) v += dpp_d<0x140>(v);
+    return v;
+}
+template <int RB>
+__device__ __forceinline__ float col_sum_f(float v) {
+    v += dpp_f<0xB1>(v);
+    v += dpp_f<0x4E>(v);
+    if constexpr (RB >= 8) v += dpp_f<0x141>(v);
+    if constexpr (RB == 16) v += dpp_f<0x140>(v);
     return v;
 }
 template <int RB, int R>
@@ -471,18 +541,30 @@ __global__ __launch_bounds__(64 * kScanWaves) void gdn_scan_kernel(const float *
     // (float) of the reference's sequential f64 sum over i < dim of cs_i x_i
     auto dot = [&](const float *x) {
         // four interleaved partial sums (the bound covers any order), then
-        // a fixed tree
-        double s4[4] = {0.0, 0.0, 0.0, 0.0}, a4[4] = {0.0, 0.0, 0.0, 0.0};
+        // a fixed tree; the absolute sum in f32 (n 2^-24 off, in the bound's
+        // room), its tree one instruction a level
+        double s4[4] = {0.0, 0.0, 0.0, 0.0};
+        float a4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const double t = (double)__fmul_rn(cs[r], x[r]);
-            s4[r & 3] += t;
-            a4[r & 3] += fabs(t);
+            const float t = __fmul_rn(cs[r], x[r]);
+            s4[r & 3] = r < 4 ? (double)t : s4[r & 3] + (double)t;
+            a4[r & 3] = __fadd_rn(a4[r & 3], fabsf(t));
         }
-        const double s = (s4[0] + s4[1]) + (s4[2] + s4[3]), ab = (a4[0] + a4[1]) + (a4[2] + a4[3]);
-        const double Sc = col_sum_d<RB>(s), Ac = col_sum_d<RB>(ab);
-        const double e = (double)(dim + 66) * 0x1p-52 * Ac;
-        const float lo = (float)(Sc - e), hi = (float)(Sc + e);
+        const double Sc = col_sum_d<RB>((s4[0] + s4[1]) + (s4[2] + s4[3]));
+        const float Ac = col_sum_f<RB>((a4[0] + a4[1]) + (a4[2] + a4[3]));
+        // Where |S| >= 2^-12 A the bound e = (dim + 67) 2^-52 A (dim <= 128) is below
+        // 2^21 units of S's last place, so with the low 29 bits of S (what f32 drops)
+        // further than that from their half both ends round alike: three integer
+        // instructions. Otherwise (about 3% of the waves) both ends are formed. (Where
+        // |S| is no normal f32, A is below 2^-114 and the sum of multiples of 2^-149 exact.)
+        float lo = (float)Sc;
+        const uint32_t low = (uint32_t)__double2loint(Sc) & 0x1FFFFFFFu;
+        const bool clear = __fmul_rn(Ac, 0x1p-12f) <= fabsf(lo) && low - (0x10000000u - 0x200000u) > 0x400000u;
+        if (!__builtin_amdgcn_ballot_w64(!clear)) return lo;
+        const double e = (double)(dim + 67) * 0x1p-52 * (double)Ac;
+        lo = (float)(Sc - e);
+        const float hi = (float)(Sc + e);
         const bool undecided = __float_as_uint(lo) != __float_as_uint(hi);
         if (!__builtin_amdgcn_ballot_w64(undecided)) return lo;
 #pragma unroll
@@ -789,7 +871,10 @@ hipError_t launch_rmsnorm_rows(float *out, int ys, const float *x, int xs, const
                            xb, xsum, z, *q8, rows, q6);
         return hipGetLastError();
     }
-    if (n <= OPS_TPB)
+    if (n <= 128 && rows >= 1024 && !xb && !xsum)  // rows enough that waves and not latency count
+        hipLaunchKernelGGL(rmsnorm_wave_kernel, dim3((rows + kNormRows - 1) / kNormRows), dim3(64 * kNormRows), 0, s, out,
+                           x, w, n, eps, xs, ys, z, rows);
+    else if (n <= OPS_TPB)
         hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(rows), dim3(OPS_TPB), 0, s, out, x, w, n, eps, xs, ys, xb, xsum, z);
     else if (n <= 4 * 1024)  // wider rows: 1024 threads, four elements each
         hipLaunchKernelGGL((rmsnorm_kernel<4, 1024>), dim3(rows), dim3(1024), 0, s, out, x, w, n, eps, xs, ys, xb, xsum,
@@ -843,9 +928,10 @@ hipError_t launch_gdn_scan(float *win, const float *kern, const float *qkv, floa
                            float eps, float scale, hipStream_t s) {
     if (!gdn_scan_ok(dim, d_conv) || n_qk < 1 || channels != (2 * n_qk + n_v) * dim) return hipErrorInvalidValue;
     if (nt == 0 || n_v == 0) return hipSuccess;
-    hipLaunchKernelGGL(gdn_conv_norm_rows_kernel, dim3((channels / dim + kConvUnits) / kConvUnits, nt),
+    const dim3 cgrid((channels / dim + kConvUnits) / kConvUnits, (nt + kConvTokens - 1) / kConvTokens);
+    hipLaunchKernelGGL(d_conv == 4 ? gdn_conv_norm_rows_kernel<4> : gdn_conv_norm_rows_kernel<0>, cgrid,
                        dim3(64 * kConvUnits), 0, s, win, kern, qkv, cv, d_conv, channels, dim, n_qk, eps, beta, gexp,
-                       dt_bias, a, n_v);
+                       dt_bias, a, n_v, nt);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // eight rows per lane: a 128-dim head on 16 lanes per column (32 waves),
