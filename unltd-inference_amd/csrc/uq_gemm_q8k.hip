@@ -685,10 +685,12 @@ hipError_t q8k_kpar_launch(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s)
 // CU (more of them hide each other's latency, at less than their number's
 // cost). The costs (us per block with 1, 2, 3 workgroups on a CU) are a least-
 // squares fit over a sweep of every shape at 17 row counts from 8 to 512 and
-// six K x N from 2048 x 700 to 12288 x 4096; the estimate is within 5% of the
-// sweep's times (standard deviation), its choice within 1.3% (Q4_K) and 0.7%
-// (Q6_K) of the best shape's in the geometric mean, where one workgroup per CU
-// as the threshold between shapes was 9% and 12% off. Examples (K x N):
+// six K x N from 2048 x 700 to 12288 x 4096 (16-row tiles at three a CU, Q4_K,
+// and the K-parallel kernel, Q6_K, then moved to the side of the line where the
+// measured best lies); the choice is within 0.3% (Q4_K) and 0.4% (Q6_K) of the
+// best shape's time in the geometric mean, 6% and 8% at worst, where one
+// workgroup per CU as the threshold between shapes was 9% and 13% off, 50% at
+// worst. Examples (K x N):
 // Q6_K 12288 x 4096 at M = 77 86 -> 68 us, at 400 218 -> 153, 4096 x 12288 at
 // 160 109 -> 73, Q4_K 4096 x 12288 at 160 86 -> 53.
 struct Q8Shape {
@@ -697,8 +699,8 @@ struct Q8Shape {
     float cost[2][3];  // [Q6_K][workgroups on the CU - 1]
 };
 constexpr Q8Shape kQ8Shapes[] = {
-    {1, 0, {1, 1}, {{0.476f, 0, 0}, {0.512f, 0, 0}}},
-    {4, 1, {3, 3}, {{0.768f, 1.102f, 1.347f}, {0.981f, 1.555f, 2.074f}}},
+    {1, 0, {1, 1}, {{0.476f, 0, 0}, {0.490f, 0, 0}}},
+    {4, 1, {3, 3}, {{0.768f, 1.102f, 1.500f}, {0.981f, 1.555f, 2.074f}}},
     {4, 2, {3, 2}, {{1.010f, 1.437f, 1.942f}, {1.214f, 1.920f, 0}}},
     {8, 2, {1, 1}, {{1.410f, 0, 0}, {1.993f, 0, 0}}},
     {8, 4, {1, 1}, {{2.270f, 0, 0}, {2.919f, 0, 0}}},
