@@ -277,8 +277,8 @@ __device__ __forceinline__ double norm_above(double sq) {
 // 16-byte load per c feeding u = 0..3; result lane l: head l >> 4, position
 // l & 15. A wave keeps its q in registers and strides over the tiles, the
 // next tile's rows in flight (16 KB a wave) while this one is multiplied.
-// Bound by reading K: 24001 positions x 4 x 256 in 26 us against 60 us for
-// the vector-unit kernel it replaces.
+// Bound by reading K: 24001 positions x 4 x 256 (98 MB) in 25.7 us against
+// 60 us for the vector-unit kernel it replaces.
 // Query z = blockIdx.z (of a prefill) sees n_ctx + z positions; its q and
 // scores are z q_st and z sc_st floats on.
 template <int HD, int GB>
@@ -714,16 +714,15 @@ struct PvStrides {
 // load) and the weight of head l & 3 (one dword). Instruction r = 0..3
 // multiplies column 4 j + r of each row: block b = (l >> 2) & 3 of it sums the
 // rows 4 k + b, so the four accumulators are independent and their blocks are
-// added at the end; result lane l: head l >> 4, column 4 (l & 3) + r. One load
-// of each kind and five conversions per 16 positions (lanes holding a column
-// each took five loads, four times the weights' bytes and eight conversions,
-// and one chain of dependent instructions: 74 us at 24001 positions of the 9B
-// shape, now 59; the 16 workgroups of 64 columns on the vector units before
-// that took 1738, replays included, against 172). A prefix is bounded by the sum over b of the blocks' |S|, A by one
-// instruction per column and 64 positions: the largest of four weights times
-// their sum of |V|. 16 columns and not 64 a workgroup: 64 workgroups at the
-// 9B shape instead of 16, with nothing to exchange between them (a caller
-// gives no workspace); the two halves of a 128-byte line on one XCD.
+// added at the end; result lane l: head l >> 4, column 4 (l & 3) + r. A prefix
+// is bounded by the sum over b of the blocks' |S|, A by one instruction per
+// column and 64 positions: the largest of four weights times their sum of |V|.
+// 16 columns and not 64 a workgroup: 64 workgroups at the 9B shape instead of
+// 16, with nothing to exchange between them (a caller gives no workspace).
+// 24001 positions of the 9B shape: 171 us with replays, 56 without; 1738 on
+// the vector units with 64 columns a workgroup. Lanes holding a column each
+// (five loads, four times the weights' bytes, eight conversions and one chain
+// of dependent instructions per 16 positions) took 74 without replays.
 constexpr int kPvWaves = 16, kPvUnroll = 4;  // 16-blocks whose loads a wave keeps in flight
 template <int G>
 __global__ __launch_bounds__(64 * kPvWaves) void attn_pv_kernel(float *__restrict__ out, const float *__restrict__ soft,
