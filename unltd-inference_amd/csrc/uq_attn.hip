@@ -985,11 +985,11 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
     };
     float sv[2][4], vv[2][4];
     const uint32_t vrow = 4 * (uint32_t)kv_len;  // bytes
-    // a block's rows as buffer loads: the block in the base, the row in the scalar offset, no
+    // a block's rows as buffer loads (any 32-bit offset): the block in the base, the row in the scalar offset, no
     // address arithmetic on the vector unit (its cycles and the f64 matrix instructions' add up)
     auto load = [&](int blk) {
-        const auto vr = __builtin_amdgcn_make_buffer_rsrc((void *)(vbase + (size_t)16 * blk * kv_len), 0, 0x7FFFFFFF, 0x00020000);
-        const auto sb = __builtin_amdgcn_make_buffer_rsrc((void *)(sbase + 16 * blk), 0, 0x7FFFFFFF, 0x00020000);
+        const auto vr = __builtin_amdgcn_make_buffer_rsrc((void *)(vbase + (size_t)16 * blk * kv_len), 0, -1, 0x00020000);
+        const auto sb = __builtin_amdgcn_make_buffer_rsrc((void *)(sbase + 16 * blk), 0, -1, 0x00020000);
 #pragma unroll
         for (int a = 0; a < 2; a++) {
             const uint4 t = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(sb, soff[a], 0, 0));
