@@ -719,8 +719,10 @@ struct PvStrides {
 // column and 64 positions: the largest of four weights times their sum of |V|.
 // 16 columns and not 64 a workgroup: 64 workgroups at the 9B shape instead of
 // 16, with nothing to exchange between them (a caller gives no workspace).
-// 24001 positions of the 9B shape: 171 us with replays, 56 without; 1738 on
-// the vector units with 64 columns a workgroup. Lanes holding a column each
+// 24001 positions of the 9B shape: 56 us without replays, 171 with those of
+// one input; 1738 on the vector units with 64 columns a workgroup. Replays
+// follow the values: scores, softmax and values together took 148 to 253 us
+// over 14 inputs, 182 in the mean. Lanes holding a column each
 // (five loads, four times the weights' bytes, eight conversions and one chain
 // of dependent instructions per 16 positions) took 74 without replays.
 constexpr int kPvWaves = 16, kPvUnroll = 4;  // 16-blocks whose loads a wave keeps in flight
