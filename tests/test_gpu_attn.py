@@ -9,6 +9,7 @@ import pytest
 
 import oracle as O
 import uq
+import uq.synth as S
 from uq import layer as L
 from uq import ops
 from test_gpu_layers import SMALL, Model
@@ -99,3 +100,47 @@ def test_attn_prefill_over_a_long_cache_equals_steps(shape, nt, pos0):
     for t in range(nt):
         assert_bitwise(got[t], ref[t], f"attn {shape} token {t} of {nt} at {pos0}")
     m.free()
+
+
+def test_attn_prefill_later_infinity_stays_out_of_earlier_tokens():
+    """Token 200's value row overflows to infinity. Tokens 192 .. 199 share
+    its pair tile, where the row meets their masked (zero) weights; the
+    reference, and the steps, read no position past a token's own."""
+    m = Model(dict(SMALL, n_head=8, n_head_kv=2, head_dim=64), seed=83)
+    c, nt, pos0, late = m.cfg, 333, 29, 200
+    nv = c.n_head_kv * c.head_dim
+    wv = S.weights(S.Q4_K, nv, c.n_embd, seed=5, sigma=0.05).reshape(-1, S.BLOCK_BYTES[S.Q4_K])
+    wv[:, 2:4] = 0  # dmin 0: an overflowing value is an infinity, never inf - inf
+    norm = m.ah["attn_norm"].copy()
+    norm[7] = 1e37
+    extra = uq.Weights(wv.reshape(-1), S.Q4_K, c.n_embd, nv), uq.DeviceArray.from_numpy(norm)
+    m.dev += extra
+    m.aw.attn_v, m.aw.attn_norm = extra
+    rng = np.random.default_rng(4)
+    X = rng.standard_normal((nt, c.n_embd)).astype(np.float32)
+    X[:, 7] = 0.0  # only the late token meets the large norm weight
+    X[late] = 0.0
+    X[late, 7] = 1.0
+    n_ctx_max = pos0 + nt
+    K, V = (rng.standard_normal((n_ctx_max, nv)).astype(np.float32) for _ in range(2))
+    ref = attn_layer(m, X[:late + 1], K, V, n_ctx_max, pos0, False)
+    got = attn_layer(m, X, K, V, n_ctx_max, pos0, True)
+    assert not np.isfinite(ref[late]).all(), "the late token's values do not overflow"
+    for t in range(late):
+        assert_bitwise(got[t], ref[t], f"attn token {t}, an infinite value row at token {late}")
+    m.free()
+
+
+@pytest.mark.parametrize("n_ctx", [40, 1100, 5000])
+def test_attn_decode_huge_values_under_underflowed_weights(n_ctx):
+    """|V| of 3e38 wherever the weight underflows to zero: finite, and zero in
+    the reference's sum, though a few such |V| added in f32 are infinite."""
+    hd = 64
+    rng = np.random.default_rng(n_ctx)
+    far = np.arange(n_ctx) % 16 == 3
+    kc = np.where(far[:, None], -3.0, 1.0).astype(np.float32) * np.ones((n_ctx, hd), np.float32)
+    vc = rng.standard_normal((n_ctx, hd)).astype(np.float32)
+    vc[far] = rng.choice([-3e38, 3e38], (int(far.sum()), hd)).astype(np.float32)
+    got = check_attn(np.ones(hd, np.float32), kc.reshape(-1), vc.reshape(-1), n_ctx, 1, 1, hd, 1.0,
+                     f"huge values n={n_ctx}", bit_exact_soft=True)
+    assert np.isfinite(got).all()

@@ -29,10 +29,12 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 
 constexpr int kAttnMaxGroup = 8;
 
+// r = lo. A NaN decides nothing, whether of S or of a bound whose parts left
+// their range: its bits may equal themselves where the reference is finite.
 __device__ __forceinline__ bool decided(double S, double e, float &r) {
     const float lo = (float)(S - e), hi = (float)(S + e);
     r = lo;
-    return __float_as_uint(lo) == __float_as_uint(hi);
+    return __float_as_uint(lo) == __float_as_uint(hi) && lo == lo;
 }
 
 // f64 sum over the lanes l, l ^ 16, l ^ 32, l ^ 48, in each of them.
@@ -374,6 +376,7 @@ __global__ __launch_bounds__(64, 2) void attn_scores_kernel(float *__restrict__ 
             float r;
             const bool ok = decided(acc[b], score_bound<HD>(qn[b], kn), r);
             unsigned long long mask = __ballot(in && !ok);
+            if (mask) mask = __ballot(in && !ok && acc[b] == acc[b]);  // a NaN of these products is the reference's
             while (mask) {
                 const int l = __ffsll(mask) - 1;
                 mask &= mask - 1;
@@ -499,6 +502,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_tile_kernel(float *__restr
             float v;
             const bool ok = decided(acc[r], score_bound<HD>(qn[r], kn), v);
             unsigned long long mask = __ballot(in && !ok);
+            if (mask) mask = __ballot(in && !ok && acc[r] == acc[r]);  // a NaN of these products is the reference's
             while (mask) {
                 const int l = __ffsll(mask) - 1;
                 mask &= mask - 1;
@@ -689,6 +693,7 @@ __device__ double lane_replay(const float *__restrict__ sr, const float *__restr
 #pragma unroll
         for (int u = 0; u < RB; u++)
             if (p0 + u < n) q += (double)sb[u] * (double)vb[u];
+        if (q != q) break;  // it stays one
     }
     return q;
 }
@@ -877,7 +882,7 @@ __global__ __launch_bounds__(64 * kPvWaves) void attn_pv_kernel(float *__restric
 #pragma unroll
         for (int u = 0; u < kPvWaves; u++)
             t.segment(part[u][w][0][lane], part[u][w][1][lane], part[u][w][2][lane], 16 * per, 16.0 + 12.0);
-        need = !decided(t.B, t.bound(), r);
+        need = !decided(t.B, t.bound(), r) && t.B == t.B;  // the sum's terms are the reference's: so is a NaN of them
     }
     if (need) {
         const int k = atomicAdd(&ntodo, 1);
@@ -1094,6 +1099,7 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
             t.segment(kh ? oS : m.S[r], kh ? oX : mX, tiny, 16 * half, 32.0 + 64.0);
             t.segment(kh ? m.S[r] : oS, kh ? mX : oX, tiny, 16 * half, 32.0 + 64.0);
             const int pr = pr0 + 16 * a + kk + 4 * r;
+            // a NaN too: positions this pair may not see took part, as zero weights, and 0 x infinity is one
             if (!decided(t.B, t.bound(), res[a][r]) && pr < pairs) {
                 need |= 1u << (4 * a + r);
                 const int k = atomicAdd(&ntodo, 1);
