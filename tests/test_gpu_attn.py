@@ -4,6 +4,8 @@ midpoints (the reference's sequential sum replayed by a workgroup), and the
 prefill's tile kernels against single-query steps over long caches. Every
 comparison is bit for bit: the kernels' contract is the reference's own bits.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -144,3 +146,88 @@ def test_attn_decode_huge_values_under_underflowed_weights(n_ctx):
     got = check_attn(np.ones(hd, np.float32), kc.reshape(-1), vc.reshape(-1), n_ctx, 1, 1, hd, 1.0,
                      f"huge values n={n_ctx}", bit_exact_soft=True)
     assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("hd,nh,nhkv", [(64, 8, 2), (256, 6, 1), (512, 2, 2)])
+def test_attn_decode_zero_rows(hd, nh, nhkv):
+    """A zero q head, zero K rows (one K row whose norm leaves the f32 range
+    beside them) and zero V columns."""
+    n_ctx = 700
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((nh, hd)).astype(np.float32)
+    K, V = (rng.standard_normal((n_ctx, nhkv, hd)).astype(np.float32) for _ in range(2))
+    q[1] = 0.0
+    K[5:40] = 0.0
+    K[11] = -0.0
+    K[300] = 1e25
+    V[:, :, 3:9] = 0.0
+    V[::2, :, 10] = -0.0
+    check_attn(q.reshape(-1), K.reshape(-1), V.reshape(-1), n_ctx, nh, nhkv, hd, 0.1, f"zero rows hd={hd}")
+
+
+def microseconds(f):
+    f()
+    best = np.inf
+    for _ in range(5):
+        uq.synchronize()
+        t = time.perf_counter()
+        for _ in range(4):
+            f()
+        uq.synchronize()
+        best = min(best, (time.perf_counter() - t) / 4)
+    return best * 1e6
+
+
+@pytest.mark.parametrize("zero", ["q", "k", "v"])
+def test_attn_decode_zero_operands_take_no_replays(zero):
+    """Scores of zero rows and sums of zero columns are decided: with the
+    scores replayed one by one a call took 1.9 times as long."""
+    n_ctx, nh, nhkv, hd = 4096, 16, 4, 256
+    rng = np.random.default_rng(1)
+    a = {n: rng.standard_normal(m).astype(np.float32) for n, m in
+         (("q", nh * hd), ("k", n_ctx * nhkv * hd), ("v", n_ctx * nhkv * hd))}
+    dout, dsoft = uq.DeviceArray(4 * nh * hd), uq.DeviceArray(4 * nh * n_ctx)
+    us = []
+    for z in (None, zero):
+        dq, dk, dv = (uq.DeviceArray.from_numpy(a[n] * np.float32(n != z)) for n in "qkv")
+        us.append(microseconds(lambda: ops.attn_decode_d(dout, dsoft, dq, dk, dv, n_ctx, nh, nhkv, hd, 0.0625)))
+        for d in (dq, dk, dv):
+            d.free()
+    print(f"random operands {us[0]:.0f} us, {zero} zero {us[1]:.0f} us", flush=True)
+    assert us[1] < 1.5 * us[0]
+
+
+@pytest.mark.parametrize("shape,nt,pos0", [
+    (dict(n_head=8, n_head_kv=2, head_dim=64), 333, 29), (dict(n_head=8, n_head_kv=2, head_dim=64), 9, 300),
+    (dict(n_embd=1024, n_v_heads=16, n_head=4, n_head_kv=1, head_dim=256), 300, 1500)])
+def test_attn_prefill_zero_operands(shape, nt, pos0):
+    """Zero tokens (q, and their own K and V rows) over a cache with zero V
+    columns and rows: the steps' bits, and about the time of other operands
+    (the values replayed, it was 6 to 8 times as much in the pair tiles)."""
+    m = Model(dict(SMALL, **shape), seed=91)
+    c = m.cfg
+    rng = np.random.default_rng(nt)
+    n_ctx_max = pos0 + nt
+    K, V = (rng.standard_normal((n_ctx_max, c.n_head_kv, c.head_dim)).astype(np.float32) for _ in range(2))
+    Z = V.copy()
+    Z[:, :, 1::2] = 0.0
+    Z[::3] = 0.0
+    X = np.zeros((nt, c.n_embd), np.float32)
+    steps = range(0, nt, max(1, nt // 40))
+    got = attn_layer(m, X, K, Z, n_ctx_max, pos0, True)
+    for t in steps:  # zero tokens: a step at each position by itself
+        own = Z.copy()
+        own[pos0:pos0 + t] = 0.0
+        assert_bitwise(got[t], attn_layer(m, X[t:t + 1], K * (np.arange(n_ctx_max) < pos0)[:, None, None], own,
+                                          n_ctx_max, pos0 + t, False)[0], f"zero token {t} of {nt}")
+    ws = uq.DeviceArray(4 * L.prefill_ws_floats(m.d, nt, attn=m.aw, n_ctx_max=n_ctx_max))
+    us = []
+    for x, v in ((rng.standard_normal(X.shape).astype(np.float32), V), (X, Z)):
+        kc, vc, dx, dl = (uq.DeviceArray.from_numpy(b) for b in (K, v, x, X))
+        us.append(microseconds(lambda: L.attn_prefill(m.d, m.aw, kc, vc, n_ctx_max, pos0, nt, dx, dl, ws)))
+        for d in (kc, vc, dx, dl):
+            d.free()
+    ws.free()
+    m.free()
+    print(f"random operands {us[0]:.0f} us, zero {us[1]:.0f} us", flush=True)
+    assert us[1] < 1.5 * us[0]

@@ -263,10 +263,25 @@ __device__ __forceinline__ double score_bound(double qn, double kn) {
     return (double)(HD + 66) * 0x1p-52 * (qn * kn);
 }
 
-// A norm from its square, at most 2^-10 above it: the f32 root, floored where
-// the square leaves the f32 range.
+// A norm from its square, at most 2^-10 above it: the f32 root, floored at
+// 2^-62 where the square leaves the f32 range, and zero for a row of zeros
+// only (any other square is at least 2^-298, whose upper word exceeds the
+// floor's bits): the score is then a zero with a bound of zero, and needs no
+// replay. Its sign may be another than the reference's, which softmax drops
+// (exp of either zero is 1).
 __device__ __forceinline__ double norm_above(double sq) {
-    return (double)fmaxf(__builtin_amdgcn_sqrtf((float)sq) * (1.0f + 0x1p-11f), 0x1p-62f);
+    const float floor = __uint_as_float(min((uint32_t)__double2hiint(sq), 0x20800000u));
+    return (double)fmaxf(__builtin_amdgcn_sqrtf((float)sq) * (1.0f + 0x1p-11f), floor);
+}
+
+// Whether a score S that the bound of the norms qn, kn left undecided needs a
+// replay. Not so, and S itself the result r: a NaN of these products, which is
+// the reference's too, and a row of zeros against one whose norm is infinite
+// in f32 (the bound is then 0 x infinity).
+__device__ __forceinline__ bool needs_replay(double S, double qn, double kn, float &r) {
+    if (S == S && qn != 0.0 && kn != 0.0) return true;
+    r = (float)S;
+    return false;
 }
 
 // scores[h][p] for a few queries (a decode step, or the first rows of a
@@ -376,7 +391,7 @@ __global__ __launch_bounds__(64, 2) void attn_scores_kernel(float *__restrict__ 
             float r;
             const bool ok = decided(acc[b], score_bound<HD>(qn[b], kn), r);
             unsigned long long mask = __ballot(in && !ok);
-            if (mask) mask = __ballot(in && !ok && acc[b] == acc[b]);  // a NaN of these products is the reference's
+            if (mask) mask = __ballot(in && !ok && needs_replay(acc[b], qn[b], kn, r));
             while (mask) {
                 const int l = __ffsll(mask) - 1;
                 mask &= mask - 1;
@@ -502,7 +517,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_tile_kernel(float *__restr
             float v;
             const bool ok = decided(acc[r], score_bound<HD>(qn[r], kn), v);
             unsigned long long mask = __ballot(in && !ok);
-            if (mask) mask = __ballot(in && !ok && acc[r] == acc[r]);  // a NaN of these products is the reference's
+            if (mask) mask = __ballot(in && !ok && needs_replay(acc[r], qn[r], kn, v));
             while (mask) {
                 const int l = __ffsll(mask) - 1;
                 mask &= mask - 1;
@@ -991,6 +1006,7 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
             }
     };
     float sv[2][4], vv[2][4];
+    uint32_t vany[2] = {0, 0};  // or of the bits of the lane's V values: is the column all zeros
     const uint32_t vrow = 4 * (uint32_t)kv_len;  // bytes
     // a block's rows as buffer loads (any 32-bit offset): the block in the base, the row in the scalar offset, no
     // address arithmetic on the vector unit (its cycles and the f64 matrix instructions' add up)
@@ -1049,6 +1065,8 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
             }
             sb[a] = bf16_4(m[0], m[1], m[2], m[3]);
             vbf[a] = bf16_4(fabsf(vv[a][0]), fabsf(vv[a][1]), fabsf(vv[a][2]), fabsf(vv[a][3]));
+            vany[a] = vany[a] | __float_as_uint(vv[a][0]) | __float_as_uint(vv[a][1]);
+            vany[a] = vany[a] | __float_as_uint(vv[a][2]) | __float_as_uint(vv[a][3]);
         }
         __builtin_amdgcn_sched_barrier(0);  // the vector work, the loads, then the matrix instructions together
         if (next < b_full) load(next);
@@ -1081,10 +1099,22 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
         if ((blk & 63) == 63) flush();
     }
     flush();
+    // bf16 products lost below the f32 range; none in a column of zeros, whose bound stays zero
+    // (a bound above a sum of zero is never decided: every output of the column would be replayed)
+    const double tiny = (double)nblk * 0x1p-121;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        vany[c] |= __shfl_xor(vany[c], 16);
+        vany[c] |= __shfl_xor(vany[c], 32);
+        if (vany[c] << 1)
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) T[a][c].A[r] += tiny;
+    }
     // wave (k, a, c) finishes its column tile k, its partner (k ^ 1, a, c) the other
     float res[2][4];
     unsigned need = 0;
-    const double tiny = (double)nblk * 0x1p-121;  // bf16 products lost below the f32 range
 #pragma unroll
     for (int a = 0; a < 2; a++) {
         const PvTile &give = kh ? T[a][0] : T[a][1], &m = kh ? T[a][1] : T[a][0];
@@ -1096,8 +1126,8 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
         for (int r = 0; r < 4; r++) {
             const double oS = xch[0][wv ^ 4][r][lane], oX = xch[1][wv ^ 4][r][lane], mX = m.PS[r] + m.A[r];
             PvErr t;
-            t.segment(kh ? oS : m.S[r], kh ? oX : mX, tiny, 16 * half, 32.0 + 64.0);
-            t.segment(kh ? m.S[r] : oS, kh ? mX : oX, tiny, 16 * half, 32.0 + 64.0);
+            t.segment(kh ? oS : m.S[r], kh ? oX : mX, 0.0, 16 * half, 32.0 + 64.0);
+            t.segment(kh ? m.S[r] : oS, kh ? mX : oX, 0.0, 16 * half, 32.0 + 64.0);
             const int pr = pr0 + 16 * a + kk + 4 * r;
             // a NaN too: positions this pair may not see took part, as zero weights, and 0 x infinity is one
             if (!decided(t.B, t.bound(), res[a][r]) && pr < pairs) {
