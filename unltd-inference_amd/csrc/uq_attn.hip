@@ -566,7 +566,10 @@ struct PvErr {
 // (the pairs D compose; all exact: multiples of q below 2^53 q), then each
 // wave in turn takes its chains of them in order, irregular runs by their
 // adds, and passes the exact sum on. 24001 positions: 110 us against 235 for
-// the adds one after another; 3071: 20 against 30.
+// the adds one after another; 3071: 20 against 30. The loop over the chains is
+// bound by its own instructions' fetch: placed anywhere, the kernel took 163 to
+// 171 us for one and the same input, by what stood before it; from the start of
+// a cache line, and with a select of the two D instead of a branch, 162.5.
 constexpr int kRun = 16;
 struct SeqLds {
     double tot[16], abs[16], dist[16], token;
@@ -669,11 +672,14 @@ __device__ __forceinline__ double wg_replay(SeqLds &L, const float *__restrict__
         for (int u = 0; u < W; u++) {
             if (w == u) {
                 unsigned long long ends = heads >> 1 | 1ull << 63;  // last lanes of the chains
+                asm volatile(".p2align 6");  // the loop below from the start of a cache line
                 while (ends) {
                     const int l = __ffsll(ends) - 1;
                     ends &= ends - 1;
                     if ((regs >> l) & 1) {
-                        s += __double2loint(s) & 1 ? lane_value(d1, l) : lane_value(d0, l);
+                        const bool odd_s = __builtin_amdgcn_readfirstlane(__double2loint(s)) & 1;
+                        const double e0 = lane_value(d0, l), e1 = lane_value(d1, l);  // both: a select, no branch
+                        s += odd_s ? e1 : e0;
                     } else {
                         double x = s;
 #pragma unroll
