@@ -103,6 +103,50 @@ def test_gdn_prefill_other_shapes_equal_steps(hd, ck, nt):
     m.free()
 
 
+def prefill_rows(m, ws, nt, n_ctx_max, name):
+    """nt rows of an array of the prefill workspace, as uq_layer.cpp lays it
+    out: the step's nodes, then the arrays in this order, each at a multiple
+    of 64 floats."""
+    c = m.cfg
+    q, kv, vd = c.n_head * c.head_dim, c.n_head_kv * c.head_dim, c.n_v_heads * c.head_dim_linear
+    off = L.ws_floats(m.d, n_ctx_max)
+    for key, row in (("xn", c.n_embd), ("qkv", m.d.channels), ("z", vd), ("beta", c.n_v_heads), ("alpha", c.n_v_heads),
+                     ("final", vd), ("qfull", 2 * q), ("k_raw", kv), ("gated", q)):
+        if key == name:
+            return ws.download(np.float32, off + row * nt)[off:].reshape(nt, row)
+        off += -(-row * nt // 64) * 64
+    raise KeyError(name)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_gdn_prefill_zero_state_under_negative_keys_gives_positive_zeros(hd):
+    """A zero state, v = 0 and every q and k below zero: all products of a
+    column are -0, and the reference's sum, which starts from +0, is +0; the
+    gated norm then carries z's sign."""
+    m = Model(dict(SMALL, head_dim_linear=hd, n_embd=8 * hd, n_head=8 * hd // 128), seed=57)
+    c, nt = m.cfg, 3
+    qk = 2 * c.n_qk_heads * hd
+    taps = np.zeros((m.d.channels, c.conv_kernel), np.float32)
+    taps[:qk, 0] = 1.0  # q, k of token t: the window's row t
+    conv = uq.DeviceArray.from_numpy(taps)
+    m.dev.append(conv)
+    m.gw.ssm_conv1d = conv
+    rng = np.random.default_rng(hd)
+    win = uq.DeviceArray.from_numpy(-1.0 - rng.random((c.conv_kernel, m.d.channels)).astype(np.float32))
+    state = uq.DeviceArray.from_numpy(np.zeros(c.n_v_heads * hd * hd, np.float32))
+    ws = uq.DeviceArray(4 * L.prefill_ws_floats(m.d, nt, gdn=m.gw))
+    dx, dl = uq.DeviceArray.from_numpy(tokens(c.n_embd, nt, 6)), uq.DeviceArray(4 * nt * c.n_embd)
+    L.gdn_prefill(m.d, m.gw, win, state, nt, dx, dl, ws)
+    uq.synchronize()
+    final, z = prefill_rows(m, ws, nt, 0, "final"), prefill_rows(m, ws, nt, 0, "z")
+    assert np.all(state.download(np.float32, state.nbytes // 4) == 0.0)
+    for t in range(nt):
+        assert_bitwise(final[t], np.copysign(np.float32(0), z[t]), f"gated output of zeros, token {t}")
+    for a in (win, state, ws, dx, dl):
+        a.free()
+    m.free()
+
+
 def attn_run(m, X, n_ctx_max, pos0, prefill, warm):
     """warm tokens by steps (positions 0 .. pos0 - 1), then X at pos0 .. by
     steps or by one prefill call; returns X's outputs and both caches."""

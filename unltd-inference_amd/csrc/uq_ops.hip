@@ -558,9 +558,11 @@ __global__ __launch_bounds__(64 * kScanWaves) void gdn_scan_kernel(const float *
         // further than that from their half both ends round alike: three integer
         // instructions. Otherwise (about 3% of the waves) both ends are formed. (Where
         // |S| is no normal f32, A is below 2^-114 and the sum of multiples of 2^-149 exact.)
+        // Not where A is 0: products that are all -0 sum to -0 here, to +0 in the reference,
+        // which starts from 0; the ends then differ and the column is replayed.
         float lo = (float)Sc;
         const uint32_t low = (uint32_t)__double2loint(Sc) & 0x1FFFFFFFu;
-        const bool clear = __fmul_rn(Ac, 0x1p-12f) <= fabsf(lo) && low - (0x10000000u - 0x200000u) > 0x400000u;
+        const bool clear = __fmul_rn(Ac, 0x1p-12f) < fabsf(lo) && low - (0x10000000u - 0x200000u) > 0x400000u;
         if (!__builtin_amdgcn_ballot_w64(!clear)) return lo;
         const double e = (double)(dim + 67) * 0x1p-52 * (double)Ac;
         lo = (float)(Sc - e);
