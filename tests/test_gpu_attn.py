@@ -1,8 +1,10 @@
 """GPU tests of the attention kernels' dispatch edges (csrc/uq_attn.hip):
 softmax rows around every row-kernel size, outputs that sit on f32 rounding
-midpoints (the reference's sequential sum replayed by a workgroup), and the
-prefill's tile kernels against single-query steps over long caches. Every
-comparison is bit for bit: the kernels' contract is the reference's own bits.
+midpoints (the reference's sequential sum replayed by a workgroup), the
+prefill's tile kernels against single-query steps over long caches and for
+every head group, undecided outputs in them, and operands that are zero, huge,
+infinite or NaN. Every comparison is bit for bit (a NaN equals a NaN): the
+kernels' contract is the reference's own bits.
 """
 import time
 
@@ -14,7 +16,8 @@ import uq
 import uq.synth as S
 from uq import layer as L
 from uq import ops
-from test_gpu_layers import SMALL, Model
+from test_gpu_layer_prefill import prefill_rows
+from test_gpu_layers import SMALL, Model, nodes_of
 from test_gpu_ops import assert_bitwise, check_attn, softmax_model
 
 pytestmark = pytest.mark.gpu
@@ -104,6 +107,81 @@ def test_attn_prefill_over_a_long_cache_equals_steps(shape, nt, pos0):
     m.free()
 
 
+def gated_rows(m, X, K, V, n_ctx_max, pos0, prefill):
+    """The attention outputs times the gates, before the output projection
+    quantizes them to eight bits, and the V cache: by one prefill or by steps."""
+    d, (nt, n) = m.d, X.shape
+    kc, vc, dx, dl = (uq.DeviceArray.from_numpy(a) for a in (K, V, X, np.zeros_like(X)))
+    ws = uq.DeviceArray(4 * max(L.ws_floats(d, n_ctx_max), L.prefill_ws_floats(d, nt, attn=m.aw, n_ctx_max=n_ctx_max)))
+    if prefill:
+        L.attn_prefill(d, m.aw, kc, vc, n_ctx_max, pos0, nt, dx, dl, ws)
+        out = prefill_rows(m, ws, nt, n_ctx_max, "gated")
+    else:
+        out = np.empty((nt, m.cfg.n_head * m.cfg.head_dim), np.float32)
+        for t in range(nt):
+            one = uq.DeviceArray.from_numpy(X[t])
+            L.attn_step(d, m.aw, kc, vc, n_ctx_max, pos0 + t, one, dl, ws)
+            out[t] = nodes_of(d, ws, ["gated"], n_ctx_max)["gated"]
+            one.free()
+    V = vc.download(np.float32, vc.nbytes // 4).reshape(n_ctx_max, m.cfg.n_head_kv, m.cfg.head_dim)
+    for a in (kc, vc, dx, dl, ws):
+        a.free()
+    return out, V
+
+
+@pytest.mark.parametrize("shape,nt,pos0", [
+    (dict(n_embd=768, n_v_heads=12, n_head=6, n_head_kv=2, head_dim=128), 301, 9),  # 3
+    (dict(n_embd=1280, n_v_heads=20, n_head=5, n_head_kv=1, head_dim=256), 250, 0),  # 5
+    (dict(n_embd=768, n_v_heads=12, n_head=12, n_head_kv=2, head_dim=64), 601, 3),  # 6
+    (dict(n_embd=1792, n_v_heads=28, n_head=7, n_head_kv=1, head_dim=256), 203, 21),  # 7
+    (dict(n_embd=1024, n_v_heads=16, n_head=8, n_head_kv=1, head_dim=128), 500, 29)])  # 8
+def test_attn_prefill_pair_tiles_of_every_head_group(shape, nt, pos0):
+    """Tokens enough for the values' pair tiles (1.4 to 2 times the rule's
+    line), groups that do not divide a tile's 64 pairs among them: a tile
+    starts and ends inside a token, the last one partly filled."""
+    m = Model(dict(SMALL, **shape), seed=101 + nt)
+    c = m.cfg
+    rng = np.random.default_rng(nt)
+    n_ctx_max = pos0 + nt + 2
+    K, V = (rng.standard_normal((n_ctx_max, c.n_head_kv, c.head_dim)).astype(np.float32) for _ in range(2))
+    X = rng.standard_normal((nt, c.n_embd)).astype(np.float32)
+    ref, _ = gated_rows(m, X, K, V, n_ctx_max, pos0, False)
+    got, _ = gated_rows(m, X, K, V, n_ctx_max, pos0, True)
+    for t in range(nt):
+        assert_bitwise(got[t], ref[t], f"attn {shape} token {t} of {nt} at {pos0}")
+    m.free()
+
+
+def test_attn_prefill_undecided_outputs_in_pair_tiles():
+    """Zero tokens weigh every position alike, and cached V columns of
+    [2^62, 1, -2^62, 1] then cancel: their sums depend on the order and no bound
+    decides them. Tokens 7 and 21, 21, 75, 105, 200, 329 put 1 to 4 pairs into
+    tiles (groups of 3: token 21 lies in two of them), times two columns of a
+    workgroup's 64 (at most eight, replayed by the workgroup) or four (each
+    lane its own), in every quarter of a tile's columns and of its pairs."""
+    m = Model(dict(SMALL, n_embd=768, n_v_heads=12, n_head=6, n_head_kv=2, head_dim=128), seed=103)
+    c, nt, pos0, zero = m.cfg, 330, 28, [7, 21, 75, 105, 200, 329]
+    planted = [(0, 5), (0, 60), (0, 64 + 19), (0, 64 + 33), (1, 0), (1, 17), (1, 33), (1, 50)]
+    rng = np.random.default_rng(8)
+    K, V = (rng.standard_normal((pos0 + nt, c.n_head_kv, c.head_dim)).astype(np.float32) for _ in range(2))
+    for kv, col in planted:
+        V[:pos0, kv, col] = np.tile(np.array([2.0 ** 62, 1.0, -(2.0 ** 62), 1.0], np.float32), pos0 // 4)
+    X = rng.standard_normal((nt, c.n_embd)).astype(np.float32)
+    X[zero] = 0.0
+    ref, _ = gated_rows(m, X, K, V, pos0 + nt, pos0, False)
+    got, after = gated_rows(m, X, K, V, pos0 + nt, pos0, True)
+    for z in zero:  # the reference's sum, its gate sigmoid(0) = 0.5
+        n = pos0 + z + 1
+        t = float(O.softmax(np.zeros(n, np.float32), 1.0)[0]) * after[:n].astype(np.float64)
+        seq = np.add.accumulate(t)[-1].astype(np.float32)
+        other = np.add.accumulate(t[::-1])[-1].astype(np.float32)
+        assert all(seq[p] != other[p] for p in planted), "another order gives the planted columns' values too"
+        assert_bitwise(got[z], np.repeat(np.float32(0.5) * seq, c.n_head // c.n_head_kv, axis=0).reshape(-1), f"zero token {z}")
+    for t in range(nt):
+        assert_bitwise(got[t], ref[t], f"attn undecided, token {t}")
+    m.free()
+
+
 def test_attn_prefill_later_infinity_stays_out_of_earlier_tokens():
     """Token 200's value row overflows to infinity. Tokens 192 .. 199 share
     its pair tile, where the row meets their masked (zero) weights; the
@@ -163,6 +241,42 @@ def test_attn_decode_zero_rows(hd, nh, nhkv):
     V[:, :, 3:9] = 0.0
     V[::2, :, 10] = -0.0
     check_attn(q.reshape(-1), K.reshape(-1), V.reshape(-1), n_ctx, nh, nhkv, hd, 0.1, f"zero rows hd={hd}")
+
+
+def test_attn_decode_infinities_and_nans():
+    """One infinite or NaN element in q, K or V of each kv head: the outputs it
+    reaches, and no others, are the reference's infinities and NaNs."""
+    n_ctx, nh, nhkv, hd = 500, 10, 5, 64
+    group = nh // nhkv
+    rng = np.random.default_rng(12)
+    q = rng.standard_normal((nh, hd)).astype(np.float32)
+    K, V = (rng.standard_normal((n_ctx, nhkv, hd)).astype(np.float32) for _ in range(2))
+    K[17, 0, 3] = np.nan  # all weights of its heads
+    V[100, 1, 5], V[200, 1, 6], V[201, 1, 7] = np.nan, np.inf, -np.inf
+    V[300, 1, 8], V[301, 1, 8] = np.inf, -np.inf
+    K[50, 2, 9] = np.inf
+    q[4, 9], q[5, 9] = -1.0, 1.0  # a weight of zero; infinity - infinity
+    V[50, 2, 4] = np.inf  # under that weight of zero
+    q[6, 1], q[7, 1] = np.nan, np.inf
+    ref, rsoft = O.attn_decode(q.reshape(-1), K.reshape(-1), V.reshape(-1), n_ctx, nh, nhkv, hd, 0.125)
+    dq, dk, dv = (uq.DeviceArray.from_numpy(a) for a in (q, K, V))
+    dout, dsoft = uq.DeviceArray(4 * nh * hd), uq.DeviceArray(4 * nh * n_ctx)
+    ops.attn_decode_d(dout, dsoft, dq, dk, dv, n_ctx, nh, nhkv, hd, 0.125)
+    uq.synchronize()
+    out, soft = dout.download(np.float32, nh * hd).reshape(nh, hd), dsoft.download(np.float32, nh * n_ctx)
+    ref, rsoft, soft = np.reshape(ref, (nh, hd)), np.reshape(rsoft, (nh, n_ctx)), soft.reshape(nh, n_ctx)
+    assert np.isnan(rsoft).any(1).tolist() == [True, True, False, False, False, True, True, True, False, False]
+    assert np.isnan(ref[2]).sum() == 2 and np.isinf(ref[2]).sum() == 2 and np.isnan(ref[4]).sum() == 1
+    for h in range(nh):
+        assert np.array_equal(np.isnan(soft[h]), np.isnan(rsoft[h])), f"head {h}: NaN weights"
+        assert np.array_equal(np.isnan(out[h]), np.isnan(ref[h])), f"head {h}: NaN outputs"
+        # softmax's expf may differ from the C library's by an ulp: the sums in order of the device's own weights
+        v = V[:, h // group].astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            seq = np.add.accumulate(soft[h].astype(np.float64)[:, None] * v)[-1].astype(np.float32)
+        ok = ~np.isnan(ref[h])
+        assert_bitwise(out[h][ok], seq[ok], f"head {h}")
+        np.testing.assert_allclose(out[h], ref[h], rtol=1e-5, atol=1e-6)
 
 
 def microseconds(f):

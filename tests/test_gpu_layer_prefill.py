@@ -211,9 +211,9 @@ def test_attn_prefill_small_equals_steps(nt, pos0, q6):
 
 @pytest.mark.parametrize("head_dim,n_head,n_head_kv", [(64, 8, 2), (512, 1, 1)])
 def test_attn_prefill_head_dims_equal_steps(head_dim, n_head, n_head_kv):
-    """Attention heads of 64 (the one-lane-per-position scores kernel at its
-    smallest tree) and of 512 (beyond it: the step's scores kernel over the
-    token dimension)."""
+    """Attention heads of 64 and of 512, the scores kernel's smallest and
+    largest (two passes over the head's dims), over the token dimension; the
+    values of 512-wide heads in pair tiles, of 64-wide ones by themselves."""
     m = Model(dict(SMALL, n_head=n_head, n_head_kv=n_head_kv, head_dim=head_dim, n_rot=32), seed=53 + head_dim)
     check_attn(m, 70, 4, n_ctx_max=128, seed=head_dim, what=f"attn head_dim={head_dim}")
     m.free()
@@ -224,9 +224,9 @@ def test_attn_prefill_head_dims_equal_steps(head_dim, n_head, n_head_kv):
     (dict(n_head=8, n_head_kv=1, head_dim=64), 19),
     (dict(n_embd=1280, n_v_heads=20, n_head=5, n_head_kv=1, head_dim=256), 23)])
 def test_attn_prefill_head_groups_equal_steps(shape, nt):
-    """Head groups of 3, 8 and 5 q heads per kv head: the prefill's pv
-    kernel takes 16 / group queries per workgroup (5, 2 and 3 here), the
-    last block of each run partly filled."""
+    """Head groups of 3, 8 and 5 q heads per kv head, few enough tokens for
+    the step's kernels over the token dimension (the pair tiles' groups are in
+    tests/test_gpu_attn.py)."""
     m = Model(dict(SMALL, **shape), seed=61 + shape["n_head"])
     check_attn(m, nt, 5, n_ctx_max=96, seed=shape["n_head"], what=f"attn {shape}")
     m.free()
