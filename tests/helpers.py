@@ -1,4 +1,6 @@
 """Shared helpers for the parity tests."""
+import time
+
 import numpy as np
 
 ATOL, RTOL = 1e-4, 1e-3  # |y - r| <= ATOL + RTOL * |r| (gemv_quant semantics)
@@ -72,3 +74,19 @@ def swiglu_bound(rg, ru):
     dsilu = sig * (1.0 + g64 * (1.0 - sig))
     tol_g, tol_u = ATOL + RTOL * np.abs(g64), ATOL + RTOL * np.abs(u64)
     return rh, ATOL + RTOL * np.abs(rh) + np.abs(dsilu * u64) * tol_g + np.abs(g64 * sig) * tol_u
+
+
+def microseconds(f):
+    """The least of five means of four calls."""
+    import uq
+
+    f()
+    best = np.inf
+    for _ in range(5):
+        uq.synchronize()
+        t = time.perf_counter()
+        for _ in range(4):
+            f()
+        uq.synchronize()
+        best = min(best, (time.perf_counter() - t) / 4)
+    return best * 1e6

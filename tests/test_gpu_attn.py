@@ -6,8 +6,6 @@ every head group, undecided outputs in them, and operands that are zero, huge,
 infinite or NaN. Every comparison is bit for bit (a NaN equals a NaN): the
 kernels' contract is the reference's own bits.
 """
-import time
-
 import numpy as np
 import pytest
 
@@ -16,6 +14,7 @@ import uq
 import uq.synth as S
 from uq import layer as L
 from uq import ops
+from helpers import microseconds
 from test_gpu_layer_prefill import prefill_rows
 from test_gpu_layers import SMALL, Model, nodes_of
 from test_gpu_ops import assert_bitwise, check_attn, softmax_model
@@ -277,19 +276,6 @@ def test_attn_decode_infinities_and_nans():
         ok = ~np.isnan(ref[h])
         assert_bitwise(out[h][ok], seq[ok], f"head {h}")
         np.testing.assert_allclose(out[h], ref[h], rtol=1e-5, atol=1e-6)
-
-
-def microseconds(f):
-    f()
-    best = np.inf
-    for _ in range(5):
-        uq.synchronize()
-        t = time.perf_counter()
-        for _ in range(4):
-            f()
-        uq.synchronize()
-        best = min(best, (time.perf_counter() - t) / 4)
-    return best * 1e6
 
 
 @pytest.mark.parametrize("zero", ["q", "k", "v"])

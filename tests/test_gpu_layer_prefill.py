@@ -22,6 +22,7 @@ import pytest
 
 import uq
 from uq import layer as L
+from helpers import microseconds
 from test_gpu_layers import FULL, SMALL, Model, assert_bitwise
 
 pytestmark = pytest.mark.gpu
@@ -145,6 +146,37 @@ def test_gdn_prefill_zero_state_under_negative_keys_gives_positive_zeros(hd):
     for a in (win, state, ws, dx, dl):
         a.free()
     m.free()
+
+
+def test_gdn_prefill_negative_zero_sums_take_no_replays():
+    """A zero state, v = 0 and q, k below zero for every token: sums of
+    products that are all -0, and of products of both signs, take the same
+    time (each of them replayed, a call took 3.9 times as long)."""
+    m = Model(dict(SMALL, head_dim_linear=128, n_embd=1024, n_head=8), seed=59)
+    c, nt = m.cfg, 512
+    qk, ck = 2 * c.n_qk_heads * 128, c.conv_kernel
+    dx, dl = uq.DeviceArray.from_numpy(np.tile(tokens(c.n_embd, 1, 7), (nt, 1))), uq.DeviceArray(4 * nt * c.n_embd)
+    ws = uq.DeviceArray(4 * L.prefill_ws_floats(m.d, nt, gdn=m.gw))
+    win = uq.DeviceArray.from_numpy(np.zeros((ck, m.d.channels), np.float32))
+    state = uq.DeviceArray.from_numpy(np.zeros(c.n_v_heads * 128 * 128, np.float32))
+    L.gdn_prefill(m.d, m.gw, win, state, nt, dx, dl, ws)
+    qkv = prefill_rows(m, ws, nt, 0, "qkv")[0]
+    us = []
+    for sign in (np.where(np.arange(qk) % 2, 1.0, -1.0), -np.ones(qk)):
+        taps = np.zeros((m.d.channels, ck), np.float32)
+        taps[:qk, ck - 1] = sign * np.sign(qkv[:qk])
+        conv = uq.DeviceArray.from_numpy(taps)
+        state.upload(np.zeros(c.n_v_heads * 128 * 128, np.float32))
+        m.gw.ssm_conv1d, own = conv, m.gw.ssm_conv1d
+        us.append(microseconds(lambda: L.gdn_prefill(m.d, m.gw, win, state, nt, dx, dl, ws)))
+        assert np.all(state.download(np.float32, state.nbytes // 4) == 0.0)
+        m.gw.ssm_conv1d = own
+        conv.free()
+    for a in (win, state, ws, dx, dl):
+        a.free()
+    m.free()
+    log(f"zeros of both signs {us[0]:.0f} us, of one {us[1]:.0f} us")
+    assert us[1] < 1.3 * us[0]
 
 
 def attn_run(m, X, n_ctx_max, pos0, prefill, warm):

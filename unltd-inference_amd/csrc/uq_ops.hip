@@ -558,15 +558,14 @@ __global__ __launch_bounds__(64 * kScanWaves) void gdn_scan_kernel(const float *
         // further than that from their half both ends round alike: three integer
         // instructions. Otherwise (about 3% of the waves) both ends are formed. (Where
         // |S| is no normal f32, A is below 2^-114 and the sum of multiples of 2^-149 exact.)
-        // Not where A is 0: products that are all -0 sum to -0 here, to +0 in the reference,
-        // which starts from 0; the ends then differ and the column is replayed.
-        float lo = (float)Sc;
+        // A zero sum is +0: -0 comes of products that are all -0 only, which the reference adds
+        // to +0; and an infinite one is the reference's, of infinite products or of finite ones.
+        const float r0 = __fadd_rn((float)Sc, 0.0f);
         const uint32_t low = (uint32_t)__double2loint(Sc) & 0x1FFFFFFFu;
-        const bool clear = __fmul_rn(Ac, 0x1p-12f) < fabsf(lo) && low - (0x10000000u - 0x200000u) > 0x400000u;
-        if (!__builtin_amdgcn_ballot_w64(!clear)) return lo;
+        const bool clear = __fmul_rn(Ac, 0x1p-12f) <= fabsf(r0) && low - (0x10000000u - 0x200000u) > 0x400000u;
+        if (!__builtin_amdgcn_ballot_w64(!clear)) return r0;
         const double e = (double)(dim + 67) * 0x1p-52 * (double)Ac;
-        lo = (float)(Sc - e);
-        const float hi = (float)(Sc + e);
+        const float lo = clear ? r0 : (float)(Sc - e), hi = clear ? r0 : (float)(Sc + e);
         const bool undecided = __float_as_uint(lo) != __float_as_uint(hi);
         if (!__builtin_amdgcn_ballot_w64(undecided)) return lo;
 #pragma unroll
