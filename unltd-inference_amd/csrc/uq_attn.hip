@@ -414,10 +414,10 @@ __global__ __launch_bounds__(64, 2) void attn_scores_kernel(float *__restrict__ 
 // LDS as f64 in the operands' order (two tiles: the next one is written while
 // this one is read, one barrier a tile). Lane l of a wave: position l & 15,
 // elements 16 c + 4 (l >> 4) + u; a 16 x 16 tile takes HD / 4 instructions of
-// 64 cycles against one 16-byte LDS read each for two of them, so the matrix
-// core is the limit: 255 queries x 16 heads over 3842 positions of 256, 16.0
-// GFLOP, take 175 us, 108 of them matrix instructions (718 us for the
-// lane-per-position vector kernel this replaces). f64 vector instructions do
+// 64 cycles against one 16-byte LDS read each for two of them: 255 queries x
+// 16 heads over 3842 positions of 256, 16.0 GFLOP, take 181 us, the matrix
+// cores busy 53% of it (58% for the next chunk's 4096 positions) and the vector
+// units 16% (718 us for the lane-per-position vector kernel this replaces). f64 vector instructions do
 // not overlap with f64 matrix ones here (4 to 7 cycles each, 16 more where the
 // kinds alternate), so the loop holds none: K and q are converted outside.
 // Query zz sees n_ctx + zz positions (causal): tiles of pairs that see none
@@ -553,7 +553,8 @@ struct PvErr {
         E += (double)(len + 4) * fabs(B) + per_block * (PS + A);
         B += S;
     }
-    // 1 + 1/32: the roundings of PS, A, E and of S +- e
+    // 1 + 1/32: the roundings of PS, E and of S +- e, and by how much an A of rounded operands may be low
+    // (attn_pv_tile_kernel: 2^-8 + 2^-12; four f32 |V| in attn_pv_kernel: less)
     __device__ __forceinline__ double bound() const { return (1.03125 * 0x1p-53) * (E + 8.0 * fabs(B)); }
 };
 
@@ -749,12 +750,14 @@ struct PvStrides {
 // column and 64 positions: the largest of four weights times their sum of |V|.
 // 16 columns and not 64 a workgroup: 64 workgroups at the 9B shape instead of
 // 16, with nothing to exchange between them (a caller gives no workspace).
-// 24001 positions of the 9B shape: 56 us without replays, 171 with those of
-// one input; 1738 on the vector units with 64 columns a workgroup. Replays
-// follow the values: scores, softmax and values together took 148 to 253 us
-// over 14 inputs, 182 in the mean. Lanes holding a column each
-// (five loads, four times the weights' bytes, eight conversions and one chain
-// of dependent instructions per 16 positions) took 74 without replays.
+// 24001 positions of the 9B shape: 56 us without replays; 1738 on the vector
+// units with 64 columns a workgroup. The 56 are spent on the 64 CUs that have a
+// workgroup: there the matrix cores are busy 20% of the time and the vector
+// units 23% (one after the other), and a wave waits for its loads 36% of its.
+// Replays follow the values: 108 to 212 us over 14 inputs, 138 in the median;
+// scores, softmax and values together 147 to 251, 182 in the mean. Lanes holding
+// a column each (five loads, four times the weights' bytes, eight conversions and
+// one chain of dependent instructions per 16 positions) took 74 without replays.
 constexpr int kPvWaves = 16, kPvUnroll = 4;  // 16-blocks whose loads a wave keeps in flight
 template <int G>
 __global__ __launch_bounds__(64 * kPvWaves) void attn_pv_kernel(float *__restrict__ out, const float *__restrict__ soft,
@@ -947,7 +950,12 @@ __device__ __forceinline__ s4 bf16_4(float a, float b, float c, float d) {
 // at positions 4 (l >> 4) + u of a 16-block, straight from memory (each
 // 16-block: 16 matrix instructions per wave against 2 + 8 loads, the next
 // block's in flight). A is bounded from above with one bf16 instruction per
-// tile and block, operands rounded up. The f64 matrix rate is the limit.
+// tile and block, the operands rounded to nearest: the sum is low by at most
+// 2^-8 of itself, and the f32 additions by 2^-12, which the 2^-5 in
+// PvErr::bound covers. 255 queries x 16 heads over 3842 positions take 195 to
+// 206 us, the matrix cores busy 52% of it and the vector units 23% (their f64
+// instructions do not overlap); a chunk over 4096 takes 223 to 237, 48% and
+// 21%: the workgroups that replay an output end last.
 // Workgroups of one pair tile (its four column blocks at hd 256) are adjacent
 // on one XCD, so the weights are read from its L2.
 constexpr int kPvTileWaves = 8;

@@ -19,18 +19,20 @@
 // Prep (gemm_q8k_prep_kernel): each row's Q8_K quantization
 // (quantize_q8_k, quants.rs:250-290) written as f16 operand octets in MFMA
 // fragment order, plus per (block, row) the f32 d and the f16 bsums.
-// Rows are padded to a multiple of 32 with zero blocks.
+// Rows are padded to a multiple of 32 (64 above 128) with zero blocks.
 //
-// Main kernel: a workgroup owns 32 rows (16 for M <= 16) x 16 NW columns,
-// one wave per 16-column tile, and walks the blocks in order (the f32
-// epilogue is sequential over blocks, so K is never split). Per block, the
-// activation octets of its rows, the raw weight blocks of its columns and
-// the rows' d / bsums stream into a two-slot LDS ring with direct-to-LDS
-// loads, issued one block ahead; one barrier per block. Each wave decodes
-// its columns' weights into B operands in registers (a lane holds column
-// lane % 16 and one octet of all eight lane sums) and keeps the eight lane
-// sums of its outputs in registers: 32 x 16 outputs fit three waves per
-// SIMD.
+// Main kernel: a workgroup owns 16, 32 or 64 rows x 16 NW columns, NW = 4 or
+// 8 waves of one 16-column tile each (q8k_shape picks), and walks the blocks
+// in order (the f32 epilogue is sequential over blocks, so K is never split
+// over workgroups; the K-parallel kernel's four waves share a 16 x 16 tile,
+// form the terms of four blocks at a time and add them in block order). Per
+// block, the activation octets of its rows, the raw weight blocks of its
+// columns and the rows' d / bsums stream into a two-slot LDS ring with
+// direct-to-LDS loads, issued one block ahead; one barrier per block. Each
+// wave decodes its columns' weights into B operands in registers (a lane
+// holds column lane % 16 and one octet of all eight lane sums) and keeps the
+// eight lane sums of its outputs in registers: 32 x 16 outputs fit three
+// waves per SIMD.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -690,19 +692,22 @@ hipError_t q8k_kpar_launch(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s)
 // measured best lies); the choice is within 0.3% (Q4_K) and 0.4% (Q6_K) of the
 // best shape's time in the geometric mean, 6% and 8% at worst, where one
 // workgroup per CU as the threshold between shapes was 9% and 13% off, 50% at
-// worst. Examples (K x N):
+// worst. Below the fit's K (256 to 1792; and up to 2047 rows, 24576 columns) the
+// choice is 2 to 5% faster than those thresholds in the geometric mean, and at
+// no size more than 5% slower (one block: 6.6 -> 6.8 us where four waves now do
+// what one did). Examples (K x N):
 // Q6_K 12288 x 4096 at M = 77 86 -> 68 us, at 400 218 -> 153, 4096 x 12288 at
 // 160 109 -> 73, Q4_K 4096 x 12288 at 160 86 -> 53.
 struct Q8Shape {
     int nw, rt;       // 16-column waves, 16-row tiles; rt 0: the K-parallel kernel, four waves per 16 x 16 tile
-    int held[2];      // workgroups a CU holds, [Q6_K]
+    int held[2];      // workgroups a CU holds, [Q6_K]; 0: not a shape of the format
     float cost[2][3];  // [Q6_K][workgroups on the CU - 1]
 };
 constexpr Q8Shape kQ8Shapes[] = {
     {1, 0, {1, 1}, {{0.476f, 0, 0}, {0.490f, 0, 0}}},
     {4, 1, {3, 3}, {{0.768f, 1.102f, 1.500f}, {0.981f, 1.555f, 2.074f}}},
     {4, 2, {3, 2}, {{1.010f, 1.437f, 1.942f}, {1.214f, 1.920f, 0}}},
-    {8, 2, {1, 1}, {{1.410f, 0, 0}, {1.993f, 0, 0}}},
+    {8, 2, {1, 0}, {{1.410f, 0, 0}, {0, 0, 0}}},  // never the least for Q6_K (1.993)
     {8, 4, {1, 1}, {{2.270f, 0, 0}, {2.919f, 0, 0}}},
 };
 template <bool Q6>
@@ -714,19 +719,22 @@ hipError_t q8k_shape(const Q8Job &j, int M, const Q8Ws &ws, hipStream_t s) {
         const Q8Shape &p = kQ8Shapes[i];
         if (p.rt == 0 && K < 8 * 256) continue;  // four blocks at a time: at least two rounds
         if (p.rt == 4 && M <= 128) continue;     // the planes' rows are padded to 32
-        if (Q6 && i == 3) continue;              // never the least for Q6_K
         const int tm = 16 * (p.rt ? p.rt : 1), held = p.held[Q6];
+        if (held == 0) continue;
         const long groups = (long)((M + tm - 1) / tm) * j.cols(16 * p.nw), q = (groups + 255) / 256;
         const float *c = p.cost[Q6];
         const float t = (float)(q / held) * c[held - 1] + (q % held ? c[q % held - 1] : 0.0f);
         if (least == 0.0f || t < least) least = t, best = i;
     }
-    switch (best) {  // 3: Q4_K only
+    switch (best) {
         case 0: return q8k_kpar_launch<Q6, 4>(j, M, ws, s);
         case 1: return q8k_launch<Q6, 4, 1>(j, M, ws, s);
         case 2: return q8k_launch<Q6, 4, 2>(j, M, ws, s);
         case 3:
-            if constexpr (!Q6) return q8k_launch<Q6, 8, 2>(j, M, ws, s);
+            if constexpr (Q6)
+                return hipErrorInvalidValue;  // held is 0
+            else
+                return q8k_launch<Q6, 8, 2>(j, M, ws, s);
         default: return q8k_launch<Q6, 8, 4>(j, M, ws, s);
     }
 }

@@ -481,7 +481,7 @@ __device__ __forceinline__ void conv_window_channel(float *__restrict__ win, con
 // for 512 tokens of a 128-dim head as single-wave workgroups, which the
 // hardware doubled up on SIMDs, as sixteen rows per lane did (288 us), and
 // 226-239 us four to a workgroup. One wave a SIMD: the instructions of a token
-// are the time. 206 us with the bound's sum in f32 and the decision mostly on
+// are the time. 210 us with the bound's sum in f32 and the decision mostly on
 // S's own bits (below).
 constexpr int kScanWaves = 4;
 template <int RB>
