@@ -104,6 +104,10 @@ def test_attn_prefill_over_a_long_cache_equals_steps(shape, nt, pos0):
     got = attn_layer(m, X, K, V, n_ctx_max, pos0, True)
     for t in range(nt):
         assert_bitwise(got[t], ref[t], f"attn {shape} token {t} of {nt} at {pos0}")
+    ref, _ = gated_rows(m, X, K, V, n_ctx_max, pos0, False)
+    got, _ = gated_rows(m, X, K, V, n_ctx_max, pos0, True)
+    for t in range(nt):
+        assert_bitwise(got[t], ref[t], f"gated attn {shape} token {t} of {nt} at {pos0}")
     m.free()
 
 
