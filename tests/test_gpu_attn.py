@@ -302,6 +302,31 @@ def test_attn_decode_zero_operands_take_no_replays(zero):
     assert us[1] < 1.5 * us[0]
 
 
+def decode_us(q, k, v, n_ctx, nh, nhkv, hd):
+    dq, dk, dv = (uq.DeviceArray.from_numpy(np.ascontiguousarray(a, np.float32)) for a in (q, k, v))
+    dout, dsoft = uq.DeviceArray(4 * nh * hd), uq.DeviceArray(4 * nh * n_ctx)
+    us = microseconds(lambda: ops.attn_decode_d(dout, dsoft, dq, dk, dv, n_ctx, nh, nhkv, hd, 0.0625))
+    for d in (dq, dk, dv, dout, dsoft):
+        d.free()
+    return us
+
+
+@pytest.mark.parametrize("qs,ks", [(1e-30, 1.0), (1.0, 1e-30), (1e-30, 1e-30), (1.0, 1e25), (1e20, 1e-5)])
+def test_attn_decode_small_and_large_operands_take_no_replays(qs, ks):
+    """Operands whose squares leave the f32 range: the bound follows them, the
+    scores are the reference's, and a call takes the time of other operands
+    (with norms in the f32 range every score was replayed)."""
+    nh, nhkv, hd = 16, 4, 256
+    rng = np.random.default_rng(3)
+    q, k, v = rng.standard_normal((nh, hd)), rng.standard_normal((4000, nhkv * hd)), rng.standard_normal((4000, nhkv * hd))
+    small = [(a * b).astype(np.float32) for a, b in ((q, qs), (k[:70], ks), (v[:70], 1.0))]
+    check_attn(*(a.reshape(-1) for a in small), 70, nh, nhkv, hd, 0.0625, f"q x {qs} k x {ks}")
+    us = decode_us(q, k, v, 4000, nh, nhkv, hd), decode_us(q * qs, k * ks, v, 4000, nh, nhkv, hd)
+    log = f"random operands {us[0]:.0f} us, q x {qs} k x {ks} {us[1]:.0f} us"
+    print(log, flush=True)
+    assert us[1] < 1.5 * us[0], log
+
+
 @pytest.mark.parametrize("shape,nt,pos0", [
     (dict(n_head=8, n_head_kv=2, head_dim=64), 333, 29), (dict(n_head=8, n_head_kv=2, head_dim=64), 9, 300),
     (dict(n_embd=1024, n_v_heads=16, n_head=4, n_head_kv=1, head_dim=256), 300, 1500)])

@@ -267,23 +267,18 @@ __device__ __forceinline__ double score_bound(double qn, double kn) {
     return (double)(HD + 66) * 0x1p-52 * (qn * kn);
 }
 
-// A norm from its square, at most 2^-10 above it: the f32 root, floored at
-// 2^-62 where the square leaves the f32 range, and zero for a row of zeros
-// only (any other square is at least 2^-298, whose upper word exceeds the
-// floor's bits): the score is then a zero with a bound of zero, and needs no
-// replay. Its sign may be another than the reference's, which softmax drops
-// (exp of either zero is 1).
-__device__ __forceinline__ double norm_above(double sq) {
-    const float floor = __uint_as_float(min((uint32_t)__double2hiint(sq), 0x20800000u));
-    return (double)fmaxf(__builtin_amdgcn_sqrtf((float)sq) * (1.0f + 0x1p-11f), floor);
-}
+// A norm from its square, at most 2^-10 above it. The root (v_sqrt_f64, 2^29
+// units in the last place) has the range of f64, where squares of f32 neither
+// underflow nor overflow. It is zero for a row of zeros: the score is then a
+// zero with a bound of zero, of another sign than the reference's perhaps,
+// which softmax drops (exp of either zero is 1).
+__device__ __forceinline__ double norm_above(double sq) { return __builtin_amdgcn_sqrt(sq) * (1.0 + 0x1p-11); }
 
-// Whether a score S that the bound of the norms qn, kn left undecided needs a
-// replay. Not so, and S itself the result r: a NaN of these products, which is
-// the reference's too, and a row of zeros against one whose norm is infinite
-// in f32 (the bound is then 0 x infinity).
+// Whether a score S that its bound left undecided needs a replay. Not so, and
+// S itself the result r: a NaN or an infinity of these products, which is the
+// reference's too, and a zero of a row of zeros.
 __device__ __forceinline__ bool needs_replay(double S, double qn, double kn, float &r) {
-    if (S == S && qn != 0.0 && kn != 0.0) return true;
+    if (S - S == 0.0 && qn != 0.0 && kn != 0.0) return true;
     r = (float)S;
     return false;
 }
