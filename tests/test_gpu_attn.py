@@ -327,6 +327,22 @@ def test_attn_decode_small_and_large_operands_take_no_replays(qs, ks):
     assert us[1] < 1.5 * us[0], log
 
 
+@pytest.mark.parametrize("n_ctx", [500, 4000])
+def test_attn_decode_infinite_values_take_no_replays(n_ctx):
+    """One infinite V row: every output is infinite, as the sum of the same
+    terms in any order is, and a call takes the time of other operands."""
+    nh, nhkv, hd = 16, 4, 256
+    rng = np.random.default_rng(4)
+    q, k, v = rng.standard_normal((nh, hd)), rng.standard_normal((n_ctx, nhkv * hd)), rng.standard_normal((n_ctx, nhkv * hd))
+    us = [decode_us(q, k, v, n_ctx, nh, nhkv, hd)]
+    v[7] = np.where(v[7] > 0, np.inf, -np.inf)
+    got = check_attn(*(a.astype(np.float32).reshape(-1) for a in (q, k, v)), n_ctx, nh, nhkv, hd, 0.0625, "infinite V row")
+    assert np.isinf(got).all()
+    us.append(decode_us(q, k, v, n_ctx, nh, nhkv, hd))
+    print(f"random operands {us[0]:.0f} us, an infinite V row {us[1]:.0f} us", flush=True)
+    assert us[1] < 1.5 * us[0]
+
+
 @pytest.mark.parametrize("shape,nt,pos0", [
     (dict(n_head=8, n_head_kv=2, head_dim=64), 333, 29), (dict(n_head=8, n_head_kv=2, head_dim=64), 9, 300),
     (dict(n_embd=1024, n_v_heads=16, n_head=4, n_head_kv=1, head_dim=256), 300, 1500)])

@@ -905,7 +905,10 @@ __global__ __launch_bounds__(64 * kPvWaves) void attn_pv_kernel(float *__restric
 #pragma unroll
         for (int u = 0; u < kPvWaves; u++)
             t.segment(part[u][w][0][lane], part[u][w][1][lane], part[u][w][2][lane], 16 * per, 16.0 + 12.0);
-        need = !decided(t.B, t.bound(), r) && t.B == t.B;  // the sum's terms are the reference's: so is a NaN of them
+        if (!decided(t.B, t.bound(), r)) {
+            need = t.B - t.B == 0.0;
+            if (!need) r = (float)t.B;  // the sum's terms are the reference's: so is a NaN or an infinity of them
+        }
     }
     if (need) {
         const int k = atomicAdd(&ntodo, 1);
@@ -1142,11 +1145,16 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
             t.segment(kh ? oS : m.S[r], kh ? oX : mX, 0.0, 16 * half, 32.0 + 64.0);
             t.segment(kh ? m.S[r] : oS, kh ? mX : oX, 0.0, 16 * half, 32.0 + 64.0);
             const int pr = pr0 + 16 * a + kk + 4 * r;
-            // a NaN too: positions this pair may not see took part, as zero weights, and 0 x infinity is one
+            // a NaN too: positions this pair may not see took part, as zero weights, and 0 x infinity is one;
+            // an infinite sum is of the pair's own terms
             if (!decided(t.B, t.bound(), res[a][r]) && pr < pairs) {
-                need |= 1u << (4 * a + r);
-                const int k = atomicAdd(&ntodo, 1);
-                if (k < kReplayMax) todo[k] = (int)threadIdx.x * 8 + 4 * a + r;
+                if (fabs(t.B) == INFINITY) {
+                    res[a][r] = (float)t.B;
+                } else {
+                    need |= 1u << (4 * a + r);
+                    const int k = atomicAdd(&ntodo, 1);
+                    if (k < kReplayMax) todo[k] = (int)threadIdx.x * 8 + 4 * a + r;
+                }
             }
         }
     }
