@@ -51,12 +51,12 @@ def midpoint_column(rng, n, w):
     return v
 
 
-@pytest.mark.parametrize("n_ctx", [40, 1000, 5000, 20000])
+@pytest.mark.parametrize("n_ctx", [40, 224, 225, 1000, 1120, 1121, 5000, 20000])
 @pytest.mark.parametrize("cols", [(5,), (0, 1, 17, 18, 63), tuple(range(16, 27))])
 def test_attn_decode_outputs_on_midpoints(n_ctx, cols):
     """Equal weights, value columns planted on f32 midpoints: no bound decides
-    them. One, a few (a workgroup replays each) and eleven of one workgroup's
-    columns (each lane its own)."""
+    them. One, a few (over more than 224 positions an output a workgroup replays
+    each) and eleven of one workgroup's columns (each lane its own)."""
     hd = 64
     rng = np.random.default_rng(n_ctx + len(cols))
     w = float(O.softmax(np.zeros(n_ctx, np.float32), 1.0)[0])
@@ -156,15 +156,17 @@ def test_attn_prefill_pair_tiles_of_every_head_group(shape, nt, pos0):
     m.free()
 
 
-def test_attn_prefill_undecided_outputs_in_pair_tiles():
+@pytest.mark.parametrize("pos0", [28, 428])
+def test_attn_prefill_undecided_outputs_in_pair_tiles(pos0):
     """Zero tokens weigh every position alike, and cached V columns of
     [2^62, 1, -2^62, 1] then cancel: their sums depend on the order and no bound
     decides them. Tokens 7 and 21, 21, 75, 105, 200, 329 put 1 to 4 pairs into
     tiles (groups of 3: token 21 lies in two of them), times two columns of a
-    workgroup's 64 (at most eight, replayed by the workgroup) or four (each
-    lane its own), in every quarter of a tile's columns and of its pairs."""
+    workgroup's 64 (at most eight, replayed by the workgroup over more than 224
+    positions) or four (each lane its own), in every quarter of a tile's columns
+    and of its pairs."""
     m = Model(dict(SMALL, n_embd=768, n_v_heads=12, n_head=6, n_head_kv=2, head_dim=128), seed=103)
-    c, nt, pos0, zero = m.cfg, 330, 28, [7, 21, 75, 105, 200, 329]
+    c, nt, zero = m.cfg, 330, [7, 21, 75, 105, 200, 329]
     planted = [(0, 5), (0, 60), (0, 64 + 19), (0, 64 + 33), (1, 0), (1, 17), (1, 33), (1, 50)]
     rng = np.random.default_rng(8)
     K, V = (rng.standard_normal((pos0 + nt, c.n_head_kv, c.head_dim)).astype(np.float32) for _ in range(2))
@@ -341,6 +343,21 @@ def test_attn_decode_infinite_values_take_no_replays(n_ctx):
     us.append(decode_us(q, k, v, n_ctx, nh, nhkv, hd))
     print(f"random operands {us[0]:.0f} us, an infinite V row {us[1]:.0f} us", flush=True)
     assert us[1] < 1.5 * us[0]
+
+
+@pytest.mark.parametrize("n_ctx", [2, 4, 16, 64])
+def test_attn_decode_midpoints_over_few_positions_replay_fast(n_ctx):
+    """A zero q over few positions weighs them by a power of two, and many sums
+    of such products end on an f32 midpoint: the lanes replay theirs side by
+    side (a workgroup, output by output, took up to 80 us more)."""
+    nh, nhkv, hd = 16, 4, 256
+    rng = np.random.default_rng(5)
+    q, k, v = rng.standard_normal((nh, hd)), rng.standard_normal((n_ctx, nhkv * hd)), rng.standard_normal((n_ctx, nhkv * hd))
+    check_attn(*(a.astype(np.float32).reshape(-1) for a in (0 * q, k, v)), n_ctx, nh, nhkv, hd, 0.0625, f"equal weights n={n_ctx}",
+               bit_exact_soft=True)
+    us = decode_us(q, k, v, n_ctx, nh, nhkv, hd), decode_us(0 * q, k, v, n_ctx, nh, nhkv, hd)
+    print(f"random q {us[0]:.0f} us, zero {us[1]:.0f} us", flush=True)
+    assert us[1] < 1.8 * us[0]
 
 
 @pytest.mark.parametrize("shape,nt,pos0", [

@@ -698,8 +698,14 @@ __device__ __forceinline__ double wg_replay(SeqLds &L, const float *__restrict__
     }
     return s;
 }
-// The same by the lane alone, its adds in order, where many outputs need it.
-constexpr int kReplayMax = 8;
+// The same by the lane alone, its adds in order, where many outputs need it or
+// the positions are few. Up to 1024 positions a workgroup takes 10 to 11 us an
+// output, one after the other; the lanes 45 ns a position, all at once: 1 and 8
+// outputs over 64 positions 11 and 80 us against 2 and 2, over 256 11 and 86
+// against 10 and 10, one over 1024 10 against 43. Few positions need it more
+// often: a sum of a few values under weights of a few bits (1/2, 1/4) may end on
+// a midpoint.
+constexpr int kReplayMax = 8, kLaneReplay = 224;
 __device__ double lane_replay(const float *__restrict__ sr, const float *__restrict__ vl, size_t kv_len, int n) {
     constexpr int RB = 16;
     double q = 0.0;
@@ -916,7 +922,7 @@ __global__ __launch_bounds__(64 * kPvWaves) void attn_pv_kernel(float *__restric
     }
     __syncthreads();
     const int nt = ntodo;
-    if (nt > kReplayMax) {
+    if (nt > kReplayMax || n_ctx <= kLaneReplay * nt) {
         if (need) r = (float)lane_replay(soft + (size_t)(kv * G + g) * n_ctx, vc + (size_t)kv * hd + i, kv_len, n_ctx);
     } else {
         for (int k = 0; k < nt; k++) {
@@ -1160,11 +1166,13 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
     }
     __syncthreads();
     const int i = col0 + 16 * kh + x, nt = ntodo;
+    // a lane takes its outputs one after the other: their number does not count here
+    const bool lanes = nt > kReplayMax || n_ctx + z_hi <= kLaneReplay;
     auto srow = [&](int pr) {
         const int zz = pr / group;
         return soft + (size_t)zz * zs.soft + (size_t)(kv * group + (pr - zz * group)) * (n_ctx + zz);
     };
-    if (nt <= kReplayMax) {
+    if (!lanes) {
         for (int k = 0; k < nt; k++) {
             const int id = todo[k] >> 3, ar = todo[k] & 7, il = id & 63, iw = id >> 6;
             const int pr = 64 * pt + 32 * ((iw >> 1) & 1) + 16 * (ar >> 2) + (il >> 4) + 4 * (ar & 3);
@@ -1184,7 +1192,7 @@ __global__ __launch_bounds__(64 * kPvTileWaves, 2) void attn_pv_tile_kernel(
             if (pr >= pairs) continue;
             const int zz = pr / group;
             float v = res[a][r];
-            if (nt > kReplayMax && ((need >> (4 * a + r)) & 1))
+            if (lanes && ((need >> (4 * a + r)) & 1))
                 v = (float)lane_replay(srow(pr), vc + (size_t)kv * hd + i, kv_len, n_ctx + zz);
             const size_t o = (size_t)(kv * group + (pr - zz * group));
             out[(size_t)zz * zs.out + o * hd + i] = v;
