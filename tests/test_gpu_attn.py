@@ -51,11 +51,11 @@ def midpoint_column(rng, n, w):
     return v
 
 
-@pytest.mark.parametrize("n_ctx", [40, 224, 225, 1000, 1120, 1121, 5000, 20000])
+@pytest.mark.parametrize("n_ctx", [40, 160, 161, 320, 321, 1000, 5000, 20000])
 @pytest.mark.parametrize("cols", [(5,), (0, 1, 17, 18, 63), tuple(range(16, 27))])
 def test_attn_decode_outputs_on_midpoints(n_ctx, cols):
     """Equal weights, value columns planted on f32 midpoints: no bound decides
-    them. One, a few (over more than 224 positions an output a workgroup replays
+    them. One, a few (over more than 160 positions an output a workgroup replays
     each) and eleven of one workgroup's columns (each lane its own)."""
     hd = 64
     rng = np.random.default_rng(n_ctx + len(cols))
@@ -162,7 +162,7 @@ def test_attn_prefill_undecided_outputs_in_pair_tiles(pos0):
     [2^62, 1, -2^62, 1] then cancel: their sums depend on the order and no bound
     decides them. Tokens 7 and 21, 21, 75, 105, 200, 329 put 1 to 4 pairs into
     tiles (groups of 3: token 21 lies in two of them), times two columns of a
-    workgroup's 64 (at most eight, replayed by the workgroup over more than 224
+    workgroup's 64 (at most eight, replayed by the workgroup over more than 160
     positions) or four (each lane its own), in every quarter of a tile's columns
     and of its pairs."""
     m = Model(dict(SMALL, n_embd=768, n_v_heads=12, n_head=6, n_head_kv=2, head_dim=128), seed=103)

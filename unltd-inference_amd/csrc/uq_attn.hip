@@ -702,10 +702,11 @@ __device__ __forceinline__ double wg_replay(SeqLds &L, const float *__restrict__
 // the positions are few. Up to 1024 positions a workgroup takes 10 to 11 us an
 // output, one after the other; the lanes 45 ns a position, all at once: 1 and 8
 // outputs over 64 positions 11 and 80 us against 2 and 2, over 256 11 and 86
-// against 10 and 10, one over 1024 10 against 43. Few positions need it more
+// against 10 and 10, one over 1024 10 against 43; 224 with 16 kv heads of 512, the
+// rows not in cache, 10 against 13, hence 160. Few positions need it more
 // often: a sum of a few values under weights of a few bits (1/2, 1/4) may end on
 // a midpoint.
-constexpr int kReplayMax = 8, kLaneReplay = 224;
+constexpr int kReplayMax = 8, kLaneReplay = 160;
 __device__ double lane_replay(const float *__restrict__ sr, const float *__restrict__ vl, size_t kv_len, int n) {
     constexpr int RB = 16;
     double q = 0.0;
